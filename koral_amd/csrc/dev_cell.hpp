@@ -91,7 +91,8 @@ KD_INL void load_geom(Geom &g, F1 src, F2 srcG)
 }
 
 // indices_21 (frames.c:2086-2106) and indices_12 (frames.c:2060-2080)
-KD_INL void lower(const double *a, double *b, const Geom &g)
+template <class GT>
+KD_INL void lower(const double *a, double *b, const GT &g)
 {
   double t[4];
 #pragma unroll
@@ -104,7 +105,8 @@ KD_INL void lower(const double *a, double *b, const Geom &g)
   for (int i = 0; i < 4; i++) b[i] = t[i];
 }
 
-KD_INL void raise_(const double *a, double *b, const Geom &g)
+template <class GT>
+KD_INL void raise_(const double *a, double *b, const GT &g)
 {
   double t[4];
 #pragma unroll
@@ -122,7 +124,8 @@ KD_INL double dot4(const double *a, const double *b)
   return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
 }
 
-KD_INL double qsq_of(double v1, double v2, double v3, const Geom &g)
+template <class GT>
+KD_INL double qsq_of(double v1, double v2, double v3, const GT &g)
 {
   const double v[4] = {0., v1, v2, v3};
   double q = 0.;
@@ -134,8 +137,9 @@ KD_INL double qsq_of(double v1, double v2, double v3, const Geom &g)
 }
 
 // VELR -> VEL4 (conv_vels_both, relele.c:105-130; core relele.c:322-338)
+template <class GT>
 KD_INL void relr_to_4vel(double v1, double v2, double v3, double *ucon, double *ucov,
-                                             const Geom &g)
+                                             const GT &g)
 {
   double qsq = qsq_of(v1, v2, v3, g);
   double gamma2 = 1. + qsq;
@@ -149,7 +153,8 @@ KD_INL void relr_to_4vel(double v1, double v2, double v3, double *ucon, double *
 }
 
 // calc_utp1 (VELR), p2u.c:548-575
-KD_INL double utp1(double v1, double v2, double v3, const Geom &g)
+template <class GT>
+KD_INL double utp1(double v1, double v2, double v3, const GT &g)
 {
   double qsq = qsq_of(v1, v2, v3, g);
   double gamma2 = 1. + qsq;
@@ -182,8 +187,8 @@ KD_INL double Sfromu(const koral_params &P, double rho, double u)
 }
 
 // p2u_mhd, p2u.c:56-159
-template <int MAG, int RAD>
-KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const Geom &g)
+template <int MAG, int RAD, class GT>
+KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const GT &g)
 {
   double gdetu = g.gdet;
   double rho = pp[0], u = pp[1];
@@ -222,8 +227,8 @@ KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const G
 }
 
 // p2u_rad (M1), p2u.c:253-307
-template <int MAG, int RAD>
-KD_INL void p2u_rad(const double *pp, double *uu, const Geom &g)
+template <int MAG, int RAD, class GT>
+KD_INL void p2u_rad(const double *pp, double *uu, const GT &g)
 {
   constexpr int EE = Lay<MAG, RAD>::EE;
   double gdetu = g.gdet;
@@ -238,8 +243,8 @@ KD_INL void p2u_rad(const double *pp, double *uu, const Geom &g)
   for (int i = 0; i < 4; i++) uu[EE + i] = gdetu * R[i];
 }
 
-template <int MAG, int RAD>
-KD_INL void p2u(const koral_params &P, const double *pp, double *uu, const Geom &g)
+template <int MAG, int RAD, class GT>
+KD_INL void p2u(const koral_params &P, const double *pp, double *uu, const GT &g)
 {
   p2u_mhd<MAG, RAD>(P, pp, uu, g);
   if (RAD) p2u_rad<MAG, RAD>(pp, uu, g);
@@ -312,23 +317,20 @@ KD_INL bool w_bad(double W, double Bsq, double QdotBsq, double Qtsq)
 // residual evaluations: the solver gives up with U2P_OVER_BUDGET, pp
 // untouched, when a point needs more (a caller that can hand the point to
 // the wave-parallel solver redoes it there from the start, same result).
+// entropy false: pp[5] is left as it was (a caller that does not read it
+// saves the two powers and the logarithm).
 //
-// WAVE: a group of WAVE_GROUP lanes (an aligned part of a wave) runs the
-// inversion of one point (uniform inputs within the group).  The two trial
-// loops of the iteration -- W *= 10 until the residual is admissible (trials
-// 0..49), and the step halving until the trial W is admissible (trials
-// 0..99) -- are searches for the first admissible trial; the lanes of the
-// group evaluate one trial each, in rounds of WAVE_GROUP trials (trial k is
-// formed with the same k sequential multiplications, or as 2^-k, which k
-// halvings of 1 give exactly), and take the first admissible one by a
-// ballot restricted to the group, which is where the sequential loop stops,
-// so the result is the same bit for bit.  A point whose iteration halves its
-// step many times then costs a few evaluations of the residual instead of
-// up to a hundred in sequence; the residual at the accepted trial also
-// serves as the next iteration's residual.  Groups of 16 lanes (four points
-// per wave) measured slower than whole waves on a torus whose deferred faces
-// need long runs of step halvings (5.9 against 4.6 ms per step), so a group
-// is the whole wave.
+// WAVE: a group of WG lanes (an aligned part of a wave) runs the inversion of
+// one point (uniform inputs within the group).  The two trial loops of the
+// iteration -- W *= 10 until the residual is admissible (trials 0..49), and
+// the step halving until the trial W is admissible (trials 0..99) -- are
+// searches for the first admissible trial; the lanes of the group evaluate
+// one trial each, in rounds of WG trials (trial k is formed with the same k
+// sequential multiplications, or as 2^-k, which k halvings of 1 give
+// exactly), and take the first admissible one by a ballot restricted to the
+// group, which is where the sequential loop stops, so the result is the same
+// bit for bit.  A point whose iteration halves its step many times then costs
+// a few evaluations of the residual instead of up to a hundred in sequence.
 #ifdef KD_HOST_CHECK
 #define KD_WAVE_SOLVER 0
 #else
@@ -337,11 +339,12 @@ KD_INL bool w_bad(double W, double Bsq, double QdotBsq, double Qtsq)
 constexpr int WAVE_GROUP = 64;  // lanes per point of the WAVE solver (divides 64)
 static_assert(64 % WAVE_GROUP == 0, "WAVE_GROUP divides the wave");
 constexpr int U2P_OVER_BUDGET = -200;
-template <int MAG, int RAD, bool WAVE = false, int WG = WAVE_GROUP>
-KD_FUN int u2p_solver_W(const koral_params &P, const double *uu, double *pp, const Geom &g, int etype,
-                        double Wstart = 0., int *iters = nullptr, int budget = 0)
+template <int MAG, int RAD, bool WAVE = false, int WG = WAVE_GROUP, class GT>
+KD_FUN int u2p_solver_W(const koral_params &P, const double *uu, double *pp, const GT &g, int etype,
+                        double Wstart = 0., int *iters = nullptr, int budget = 0, bool entropy = true)
 {
   static_assert(64 % WG == 0, "a lane group divides the wave");
+  constexpr bool GROUP = WAVE && KD_WAVE_SOLVER;  // a host build runs the sequential loop
   double gdetu = g.gdet;
   double alpha = sqrt(-1. / g.G[0][0]);
   double D = uu[0] / gdetu * alpha;
@@ -386,127 +389,133 @@ KD_FUN int u2p_solver_W(const koral_params &P, const double *uu, double *pp, con
 
   double gamma2 = 1. + qsq_of(pp[2], pp[3], pp[4], g);
   double W = Wstart > 0. ? Wstart : (pp[0] + P.gamma * pp[1]) * gamma2;
-  double f0, dfdW, err;
-  int i_increase = 0;
-  int nev = 0;  // residual evaluations of the sequential path (budget)
   if (iters) *iters = 0;
+  // One evaluation of the residual per trip of the loop: at the start W and
+  // its bumps (SEARCH), at a step and its halvings (STEP), or at the W a
+  // vanishing derivative moved to (MOVED).  An admissible trial's residual is
+  // the next iteration's residual at W (same inputs, same values).
+  enum { SEARCH, STEP, MOVED } phase = SEARCH;
+  double Wt = W, f0 = 0., dfdW = 0., err = 0., dumpfac = 1.;
+  int iter = 0;
+  int k0 = 0;   // trials of the phase rejected so far
+  int nev = 0;  // eighths of a residual evaluation spent by the sequential path (budget)
+  // The step halved to the fraction h = 2^-k of f0 / dfdW: W - h f0 / dfdW,
+  // formed from the quotient where scaling by a power of two is exact (no
+  // quotient near the ends of the exponent range), so that a halving costs no
+  // division.
+  double step = 0.;
+  bool exact_scaling = false;
+  auto halved = [&](double h) { return exact_scaling ? W - h * step : W - h * f0 / dfdW; };
 #if KD_WAVE_SOLVER
-  if constexpr (WAVE) {
-    const int lane = threadIdx.x & 63, sub = lane % WG, g0 = lane - sub;
-    const unsigned long long gmask = (WG == 64) ? ~0ull : (((1ull << WG) - 1ull) << g0);
-    bool found = false;
-    for (int r = 0; r * WG < 50 && !found; r++) {
-      const int k = r * WG + sub;
-      double Wk = W;
-      for (int q = 0; q < k; q++) Wk *= 10.;
-      bool ok = false;
-      if (k < 50) {
-        double f = 0., df = 0., e;
-        f_u2p(P, etype, Wk - D, c, f, df, e);
-        ok = !(w_bad(Wk, Bsq, QdotBsq, Qtsq) || !isfinite(f) || !isfinite(df));
+  const int sub = threadIdx.x & (WG - 1), g0 = (threadIdx.x & 63) - sub;
+  const unsigned long long gmask = (WG == 64) ? ~0ull : (((1ull << (WG & 63)) - 1ull) << g0);
+#endif
+  for (;;) {
+    const int kmax = phase == STEP ? 100 : 50;
+    double f = 0., df = 0., e = 0.;
+    bool ok;
+#if KD_WAVE_SOLVER
+    if constexpr (GROUP) {
+      const int k = k0 + sub;
+      Wt = W;
+      if (phase == STEP) {
+        // k halvings of 1 are exact: 2^-k
+        Wt = halved(ldexp(1., -k));
+      } else if (phase == SEARCH) {
+        for (int q = 0; q < k; q++) Wt *= 10.;
+      }
+      ok = k < kmax && (phase == MOVED || !w_bad(Wt, Bsq, QdotBsq, Qtsq));
+      if (ok) {
+        f_u2p(P, etype, Wt - D, c, f, df, e);
+        ok = phase == MOVED || (isfinite(f) && isfinite(df));
       }
       const unsigned long long m = __ballot(ok) & gmask;
-      if (m) {
-        W = __shfl(Wk, __ffsll(m) - 1);
-        found = true;
+      ok = m != 0;
+      if (ok) {
+        const int win = __ffsll(m) - 1;
+        Wt = __shfl(Wt, win);
+        f = __shfl(f, win);
+        df = __shfl(df, win);
+        e = __shfl(e, win);
       }
-    }
-    if (!found) return -150;
-  } else
-#endif
-  {
-    for (;;) {
-      f0 = dfdW = 0.;
-      if (budget > 0 && ++nev > budget) return U2P_OVER_BUDGET;
-      f_u2p(P, etype, W - D, c, f0, dfdW, err);
-      if ((w_bad(W, Bsq, QdotBsq, Qtsq) || !isfinite(f0) || !isfinite(dfdW)) && i_increase < 50) {
-        W *= 10.;
-        i_increase++;
-        continue;
-      }
-      break;
-    }
-    if (i_increase >= 50) return -150;
-  }
-  int iter = 0;
-  double Wprev;
-  // WAVE: the residual at the accepted trial, evaluated by the winning lane,
-  // is the next iteration's residual at W (same inputs, same values).  The
-  // sequential path evaluates it again: carrying it there lengthened
-  // register lifetimes in the register-bound implicit kernels (3 % slower).
-  bool have = false;
-  double fc = 0., dfc = 0., ec = 0.;
-  do {
-    Wprev = W;
-    iter++;
-    if (iters) *iters = iter;
-    if (WAVE && have) {
-      f0 = fc;
-      dfdW = dfc;
-      err = ec;
-    } else {
-      if (budget > 0 && ++nev > budget) return U2P_OVER_BUDGET;
-      f_u2p(P, etype, W - D, c, f0, dfdW, err);
-    }
-    have = false;
-    if (err < P.u2pconv) break;
-    if (dfdW == 0.) {
-      W *= 1.1;
-      continue;
-    }
-    double Wnew = W - f0 / dfdW;
-#if KD_WAVE_SOLVER
-    if constexpr (WAVE) {
-      // trials k = 0..99 in rounds of WG; trial k halves the step k times
-      const int lane = threadIdx.x & 63, sub = lane % WG, g0 = lane - sub;
-      const unsigned long long gmask = (WG == 64) ? ~0ull : (((1ull << WG) - 1ull) << g0);
-      int found = -1;
-      for (int round = 0; round * WG < 100 && found < 0; round++) {
-        const int k = round * WG + sub;
-        // k halvings of 1 are exact: 2^-k
-        const double dumpfac = ldexp(1., -k);
-        const double Wt = k == 0 ? Wnew : W - dumpfac * f0 / dfdW;
-        bool ok = false;
-        double f0t = 0., dft = 0., errt = 0.;
-        if (k < 100) {
-          f_u2p(P, etype, Wt - D, c, f0t, dft, errt);
-          ok = !(w_bad(Wt, Bsq, QdotBsq, Qtsq) || !isfinite(f0t) || !isfinite(dft));
-        }
-        const unsigned long long m = __ballot(ok) & gmask;
-        if (m) {
-          const int win = __ffsll(m) - 1;
-          found = round * WG + win - g0;
-          Wnew = __shfl(Wt, win);
-          fc = __shfl(f0t, win);
-          dfc = __shfl(dft, win);
-          ec = __shfl(errt, win);
-          have = true;
-        }
-      }
-      if (found < 0) return -101;
     } else
 #endif
     {
-      int idump = 0;
-      double dumpfac = 1.;
-      for (;;) {
-        double f0t = 0., dft = 0., errt;
-        if (budget > 0 && ++nev > budget) return U2P_OVER_BUDGET;
-        f_u2p(P, etype, Wnew - D, c, f0t, dft, errt);
-        if ((w_bad(Wnew, Bsq, QdotBsq, Qtsq) || !isfinite(f0t) || !isfinite(dft)) && idump < 100) {
-          idump++;
-          dumpfac /= 2.;
-          Wnew = W - dumpfac * f0 / dfdW;
-          continue;
-        }
-        break;
+      // A W with v^2 >= 1 is inadmissible whatever the residual: bumps and
+      // halvings out of that range take the cheap test alone, and nearly
+      // every rejection is one of these.  Four halvings are tested at a time
+      // (they are independent; up to 54 follow one another where the step
+      // points out of the range for good).
+      while (phase == SEARCH && w_bad(Wt, Bsq, QdotBsq, Qtsq)) {
+        if (++k0 >= kmax) return -150;
+        nev++;
+        Wt *= 10.;
       }
-      if (idump >= 100) return -101;
+      while (phase == STEP && w_bad(Wt, Bsq, QdotBsq, Qtsq)) {
+        int first = 4;
+        double t[4];
+#pragma unroll
+        for (int q = 3; q >= 0; q--) {
+          t[q] = halved(dumpfac * (q == 0 ? .5 : q == 1 ? .25 : q == 2 ? .125 : .0625));
+          if (!w_bad(t[q], Bsq, QdotBsq, Qtsq)) first = q;
+        }
+        const int m = first < 4 ? first : 3;
+        k0 += m + 1;
+        if (k0 >= kmax) return -101;
+        nev++;
+        dumpfac *= m == 0 ? .5 : m == 1 ? .25 : m == 2 ? .125 : .0625;
+        Wt = m == 0 ? t[0] : m == 1 ? t[1] : m == 2 ? t[2] : t[3];
+      }
+      nev += 8;
+      if (budget > 0 && nev > 8 * budget) return U2P_OVER_BUDGET;
+      f_u2p(P, etype, Wt - D, c, f, df, e);
+      ok = phase == MOVED || (isfinite(f) && isfinite(df));
     }
-    W = Wnew;
-    if (fabs(W) > BIG) return -103;
-    if (fabs((W - Wprev) / Wprev) < P.u2pconv && err < 1.e-1) break;
-  } while (iter < 50);
+    if (!ok) {
+      k0 += GROUP ? WG : 1;
+      if (k0 >= kmax) return phase == STEP ? -101 : -150;
+      if (!GROUP) {
+        dumpfac *= .5;
+        Wt = phase == STEP ? halved(dumpfac) : Wt * 10.;
+      }
+      continue;
+    }
+    if (phase == STEP) {
+      const double Wprev = W;
+      W = Wt;
+      if (fabs(W) > BIG) return -103;
+      if (fabs((W - Wprev) / Wprev) < P.u2pconv && err < 1.e-1) break;
+      if (iter >= 50) break;
+      // A step halved away to nothing (some 54 halvings) with an error too
+      // large to stop at: W, its residual and so every further iteration
+      // repeat this one, until the iterations run out.
+      if (W == Wprev) {
+        if (iters) *iters = 50;
+        return -102;
+      }
+    } else {
+      W = Wt;
+    }
+    iter++;
+    if (iters) *iters = iter;
+    f0 = f;
+    dfdW = df;
+    err = e;
+    if (err < P.u2pconv) break;
+    k0 = 0;
+    if (dfdW == 0.) {
+      W *= 1.1;
+      if (iter >= 50) break;
+      Wt = W;
+      phase = MOVED;
+      continue;
+    }
+    step = f0 / dfdW;
+    exact_scaling = fabs(f0) > 1e-250 && fabs(step) > 1e-250 && fabs(step) < 1e290;
+    Wt = W - step;
+    dumpfac = 1.;
+    phase = STEP;
+  }
   if (iter >= 50) return -102;
   if (!isfinite(W)) return -103;
 
@@ -528,7 +537,7 @@ KD_FUN int u2p_solver_W(const koral_params &P, const double *uu, double *pp, con
   pp[3] = ut2;
   pp[4] = ut3;
   if (rho < 0.) return -105;
-  pp[5] = Sfromu(P, rho, uint);
+  if (entropy) pp[5] = Sfromu(P, rho, uint);
   if (MAG) {
     pp[6] = uu[6] / gdetu;
     pp[7] = uu[7] / gdetu;
@@ -540,7 +549,8 @@ KD_FUN int u2p_solver_W(const koral_params &P, const double *uu, double *pp, con
 // ---------------------------------------------------------------------------
 // M1 closure inversion, u2prad.c:9-481
 // ---------------------------------------------------------------------------
-KD_INL void m1_inv(const double *Av, const Geom &g, double &S, double &Sig)
+template <class GT>
+KD_INL void m1_inv(const double *Av, const GT &g, double &S, double &Sig)
 {
   S = g.G[0][1] * Av[1] + g.G[0][2] * Av[2] + g.G[0][3] * Av[3];
   double q = 0.;
@@ -551,40 +561,32 @@ KD_INL void m1_inv(const double *Av, const Geom &g, double &S, double &Sig)
   Sig = q;
 }
 
-// get_m1closure_gammarel2_cold, u2prad.c:9-102
-KD_INL void m1_cold(const Geom &g, const double *Avc_in, double gammarel2, double &Av0,
-                                        double &Erf, double *urf)
+// The two roots of get_m1closure_gammarel2_cold (u2prad.c:9-102) up to the
+// time component Av0 of the momentum they stand for: x = gamma^2 / alpha^2
+KD_INL void m1_cold(double gtt, double S, double SS, double x, double &tt, double &q4, double &rt, double &Av0)
 {
-  double alpha = g.alpha;
-  double x = gammarel2 / (alpha * alpha);
-  double gtt = g.G[0][0];
-  double S, Sig;
-  m1_inv(Avc_in, g, S, Sig);
-  double SS = S * S - gtt * Sig;
-  double tt = x * (gtt + x);
-  double q4 = gtt + 4. * x;
-  double rt = sqrt(SS * tt * q4 * q4);
+  tt = x * (gtt + x);
+  q4 = gtt + 4. * x;
+  rt = sqrt(SS * tt * q4 * q4);
   Av0 = 0.25 * (-4. * S * tt + rt) / (gtt * tt);
-  Erf = 0.75 * rt / (tt * q4);
-  double Avcov[4] = {Av0, Avc_in[1], Avc_in[2], Avc_in[3]}, Avcon[4];
-  raise_(Avcov, Avcon, g);
-  double grel = sqrt(gammarel2);
-#pragma unroll
-  for (int j = 1; j < 4; j++)
-    urf[j] = (Erf > 0.0) ? alpha * (Avcon[j] + 1. / 3. * Erf * g.G[0][j] * (4.0 * gammarel2 - 1.0)) /
-                               (4. / 3. * Erf * grel)
-                         : 0.0;
 }
 
-template <int MAG, int RAD>
-KD_FUN int u2p_rad(const koral_params &P, const double *uu, double *pp, const Geom &g, int &corrected)
+// A state with no admissible root takes the slow (gamma^2 = (1 + 10 eps)^2) or
+// the fast (GAMMAMAXRAD^2) cold one, whichever Av0 is nearer.  Only that
+// root's energy and velocities are formed, by the expressions an admissible
+// root goes through, which both kinds of lane share: the few failing lanes a
+// wave of states nearly always holds cost it two Av0 instead of two complete
+// roots beside its own.
+template <int MAG, int RAD, class GT>
+KD_FUN int u2p_rad(const koral_params &P, const double *uu, double *pp, const GT &g, int &corrected)
 {
   constexpr int EE = Lay<MAG, RAD>::EE;
   double gdetu = g.gdet;
   corrected = 0;
   double Avcov[4] = {uu[EE] / gdetu, uu[EE + 1] / gdetu, uu[EE + 2] / gdetu, uu[EE + 3] / gdetu};
-  double Avcon[4];
-  raise_(Avcov, Avcon, g);
+  double Avcon0 = 0.;
+#pragma unroll
+  for (int k = 0; k < 4; k++) Avcon0 += Avcov[k] * g.G[0][k];
   double alpha = g.alpha;
   double gtt = g.G[0][0];
   double S, Sig;
@@ -598,38 +600,40 @@ KD_FUN int u2p_rad(const koral_params &P, const double *uu, double *pp, const Ge
   if (gamma2 < GAMMASMALLLIMIT || !isfinite(gamma2)) gamma2 = (-base + R * sq) / (4. * Q);
   double gammarel2 = gamma2 * alpha * alpha;
   if (gammarel2 > GAMMASMALLLIMIT && gammarel2 < 1.0) gammarel2 = 1.0;
-  double Erf = 3. * Avcon[0] * alpha * alpha / (4. * gammarel2 - 1.0);
+  double Erf = 3. * Avcon0 * alpha * alpha / (4. * gammarel2 - 1.0);
   double gmax = P.gammamaxrad;
-  double u1, u2, u3;
   bool nonfailure = gammarel2 >= 1.0 && Erf > P.eradfloor &&
                     gammarel2 <= gmax * gmax / GAMMASMALLLIMIT / GAMMASMALLLIMIT;
-  if (nonfailure) {
-    double grel = sqrt(gammarel2);
-    u1 = alpha * (Avcon[1] + 1. / 3. * Erf * g.G[0][1] * (4.0 * gammarel2 - 1.0)) / (4. / 3. * Erf * grel);
-    u2 = alpha * (Avcon[2] + 1. / 3. * Erf * g.G[0][2] * (4.0 * gammarel2 - 1.0)) / (4. / 3. * Erf * grel);
-    u3 = alpha * (Avcon[3] + 1. / 3. * Erf * g.G[0][3] * (4.0 * gammarel2 - 1.0)) / (4. / 3. * Erf * grel);
-  } else {
-    double g2slow = kd_pow(1.0 + 10.0 * DBL_EPSILON, 2.0);
-    double g2fast = gmax * gmax;
-    double As, Es, us[4] = {0., 0., 0., 0.}, Af, Ef, uf[4] = {0., 0., 0., 0.};
-    m1_cold(g, Avcov, g2slow, As, Es, us);
-    m1_cold(g, Avcov, g2fast, Af, Ef, uf);
-    if (fabs(As - Avcov[0]) > fabs(Af - Avcov[0])) {
-      u1 = uf[1]; u2 = uf[2]; u3 = uf[3];
-      gammarel2 = g2fast;
-      Erf = Ef;
-    } else {
-      u1 = us[1]; u2 = us[2]; u3 = us[3];
-      gammarel2 = g2slow;
-      Erf = Es;
-    }
+  if (!nonfailure) {
+    const double g2slow = (1.0 + 10.0 * DBL_EPSILON) * (1.0 + 10.0 * DBL_EPSILON);
+    const double g2fast = gmax * gmax;
+    const double SS = S * S - gtt * Sig;
+    double ts, qs, rs, As, tf, qf, rf, Af;
+    m1_cold(gtt, S, SS, g2slow / (alpha * alpha), ts, qs, rs, As);
+    m1_cold(gtt, S, SS, g2fast / (alpha * alpha), tf, qf, rf, Af);
+    const bool fast = fabs(As - Avcov[0]) > fabs(Af - Avcov[0]);
+    gammarel2 = fast ? g2fast : g2slow;
+    const double tt = fast ? tf : ts, q4 = fast ? qf : qs, rt = fast ? rf : rs;
+    Erf = 0.75 * rt / (tt * q4);
+    Avcov[0] = fast ? Af : As;
     corrected = 1;
-    if (!isfinite(Erf) || !isfinite(gammarel2) || !isfinite(u1) || !isfinite(u2) || !isfinite(u3)) return -1;
   }
+  double u[3];
+  const double grel = sqrt(gammarel2);
+#pragma unroll
+  for (int j = 1; j < 4; j++) {
+    double Av = 0.;
+#pragma unroll
+    for (int k = 0; k < 4; k++) Av += Avcov[k] * g.G[j][k];
+    const double v = alpha * (Av + 1. / 3. * Erf * g.G[0][j] * (4.0 * gammarel2 - 1.0)) / (4. / 3. * Erf * grel);
+    u[j - 1] = (nonfailure || Erf > 0.0) ? v : 0.0;
+  }
+  if (!nonfailure && (!isfinite(Erf) || !isfinite(u[0]) || !isfinite(u[1]) || !isfinite(u[2]) || !isfinite(gammarel2)))
+    return -1;
   pp[EE] = Erf;
-  pp[EE + 1] = u1;
-  pp[EE + 2] = u2;
-  pp[EE + 3] = u3;
+  pp[EE + 1] = u[0];
+  pp[EE + 2] = u[1];
+  pp[EE + 3] = u[2];
   return 0;
 }
 
@@ -637,8 +641,8 @@ KD_FUN int u2p_rad(const koral_params &P, const double *uu, double *pp, const Ge
 // radiation field and four-force
 // ---------------------------------------------------------------------------
 // calc_Rij_M1, rad.c:1944-1975
-template <int MAG, int RAD>
-KD_INL void Rij_M1(const double *pp, const Geom &g, double R[4][4])
+template <int MAG, int RAD, class GT>
+KD_INL void Rij_M1(const double *pp, const GT &g, double R[4][4])
 {
   constexpr int EE = Lay<MAG, RAD>::EE;
   double E = pp[EE];
@@ -670,10 +674,13 @@ KD_INL double kappa_abs(const koral_params &P, double rho, double u)
 
 KD_INL double kappa_es(const koral_params &P, double rho) { return P.kappa_es_coef * rho; }
 
-// calc_Gi, rad.c:1787-1888
-template <int MAG, int RAD>
-KD_INL void calc_Gi(const koral_params &P, const double *pp, const Geom &g, double *Gi,
-                                        int labframe)
+// calc_Gi, rad.c:1787-1888, in the lab frame; with FFP the fluid-frame
+// quantities of the same state as well: its time component Gff there
+// (labframe 0), and Rtt and u^t of calc_ff_Rtt (rad.c:2833-2862), which take
+// the same R^ij and velocities
+template <int MAG, int RAD, bool FFP, class GT>
+KD_INL void calc_Gi_ff(const koral_params &P, const double *pp, const GT &g, double *Gi, bool ff, double &Gff,
+                       double &Rtt, double &ut)
 {
   double R[4][4];
   Rij_M1<MAG, RAD>(pp, g, R);
@@ -697,12 +704,35 @@ KD_INL void calc_Gi(const koral_params &P, const double *pp, const Geom &g, doub
     for (int j = 0; j < 4; j++) Ru += R[i][j] * ucov[j];
     Gi[i] = -(kappa + kes) * Ru - (kes * Ruu + kappa * 4. * PI_KORAL * B) * ucon[i];
   }
-  if (labframe == 0) Gi[0] = -kappa * 4. * PI_KORAL * B + kappa * Ruu;
+  if (FFP && ff) {
+    Gff = -kappa * 4. * PI_KORAL * B + kappa * Ruu;
+    ut = ucon[0];
+    Rtt = 0.;
+#pragma unroll
+    for (int i1 = 0; i1 < 4; i1++) {
+#pragma unroll
+      for (int i2 = 0; i2 < 4; i2++) {
+        double Rm = 0.;
+#pragma unroll
+        for (int k = 0; k < 4; k++) Rm += R[i1][k] * g.g[k][i2];
+        Rtt += -Rm * ucon[i2] * ucov[i1];
+      }
+    }
+  }
+}
+
+template <int MAG, int RAD>
+KD_INL void calc_Gi(const koral_params &P, const double *pp, const Geom &g, double *Gi,
+                                        int labframe)
+{
+  double Gff = 0., Rtt, ut;
+  calc_Gi_ff<MAG, RAD, true>(P, pp, g, Gi, labframe == 0, Gff, Rtt, ut);
+  if (labframe == 0) Gi[0] = Gff;
 }
 
 // calc_ff_Rtt, rad.c:2833-2862
-template <int MAG, int RAD>
-KD_INL double ff_Rtt(const double *pp, const Geom &g, double *ucon_out)
+template <int MAG, int RAD, class GT>
+KD_INL double ff_Rtt(const double *pp, const GT &g, double *ucon_out)
 {
   double uc[4], uv[4];
   relr_to_4vel(pp[2], pp[3], pp[4], uc, uv, g);
