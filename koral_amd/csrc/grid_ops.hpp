@@ -1406,7 +1406,7 @@ inline long face_states_cap(const DGrid &G)
 // allocates exactly these (koral_hip_grid_create); the host check of the
 // operators allocates the same sizes behind guard pages.  Directions that are
 // collapsed get no flux, face-state or floor-list buffers.
-constexpr int IMP_LIST_COUNTERS = 32;
+constexpr int IMP_LIST_COUNTERS = 33;
 template <class F>
 void grid_buffers(GridBufs &s, F &&f)
 {

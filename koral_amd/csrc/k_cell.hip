@@ -196,15 +196,28 @@ struct BatchCells {
   }
   __device__ __forceinline__ void init(long c) const { info[5 * n + c] = 0; }
   __device__ __forceinline__ void add_iters(long c, int it) const { info[5 * n + c] += it; }
-  __device__ __forceinline__ void done_ok(long c, const double *u, const double *p, int iters, int attempt, int wp,
-                                          int we, int wf) const
+  __device__ __forceinline__ bool solved(long c) const { return info[1 * n + c] >= 0; }
+  __device__ __forceinline__ void load_p(long c, double *p, Geom &g) const
+  {
+    constexpr int NV = Lay<MAG, RAD>::NV;
+    load_point<MAG, RAD>(g20, G20, n, c, g);
+#pragma unroll
+    for (int v = 0; v < NV; v++) p[v] = pp[v * n + c];
+  }
+  __device__ __forceinline__ void finish(long c, const double *p, const double *u) const
+  {
+    constexpr int NV = Lay<MAG, RAD>::NV;
+    pp[5 * n + c] = p[5];
+#pragma unroll
+    for (int v = 0; v < NV; v++) uu[v * n + c] = u[v];
+  }
+  __device__ __forceinline__ void done_ok(long c, const double *p, int iters, int attempt, int wp, int we,
+                                          int wf) const
   {
     constexpr int NV = Lay<MAG, RAD>::NV;
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      pp[v * n + c] = p[v];
-      uu[v * n + c] = u[v];
-    }
+    for (int v = 0; v < NV; v++)
+      if (v != 5) pp[v * n + c] = p[v];
     flags[F_RADSOURCETYPE * n + c] = 3;
     flags[F_RADFIXUP * n + c] = 0;
     flags[F_RADIMPFIXUP * n + c] = 0;

@@ -137,19 +137,39 @@ struct GridCells {
     int ix, iy;
     const long c = cell(i, ix, iy);
     geom_cell(G, ix, iy, g);
-    load_p<MAG, 1>(p, G.ncell, c, pp00);
-    load_p<MAG, 1>(u, G.ncell, c, uu00);
+    kd::load_p<MAG, 1>(p, G.ncell, c, pp00);
+    kd::load_p<MAG, 1>(u, G.ncell, c, uu00);
     dtc = clk[1] * fac;
   }
   __device__ __forceinline__ void init(long) const {}
   __device__ __forceinline__ void add_iters(long, int) const {}
-  __device__ __forceinline__ void done_ok(long i, const double *uu, const double *pp, int, int, int, int,
-                                          int) const
+  __device__ __forceinline__ bool solved(long i) const
+  {
+    int ix, iy;
+    return fl[F_RADIMPFIXUP * G.ncell + cell(i, ix, iy)] == 0;
+  }
+  __device__ __forceinline__ void load_p(long i, double *pp, Geom &g) const
+  {
+    int ix, iy;
+    const long c = cell(i, ix, iy);
+    geom_cell(G, ix, iy, g);
+    kd::load_p<MAG, 1>(p, G.ncell, c, pp);
+  }
+  __device__ __forceinline__ void finish(long i, const double *pp, const double *uu) const
   {
     int ix, iy;
     const long c = cell(i, ix, iy), n = G.ncell;
-    store_p<MAG, 1>(p, n, c, pp);
+    p[5 * n + c] = pp[5];
     store_p<MAG, 1>(u, n, c, uu);
+  }
+  __device__ __forceinline__ void done_ok(long i, const double *pp, int, int, int, int, int) const
+  {
+    constexpr int NV = Lay<MAG, 1>::NV;
+    int ix, iy;
+    const long c = cell(i, ix, iy), n = G.ncell;
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+      if (v != 5) p[v * n + c] = pp[v];
     fl[F_RADSOURCETYPE * n + c] = 3;
     fl[F_RADFIXUP * n + c] = 0;
     fl[F_RADIMPFIXUP * n + c] = 0;
