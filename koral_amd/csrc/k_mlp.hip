@@ -20,8 +20,7 @@
 // asinh((x*_i - x0_i) / VSCALE) for the three velocity components.
 #include <hip/hip_runtime.h>
 #include <math.h>
-#include <mutex>
-#include <vector>
+#include <type_traits>
 #include "koral_hip.h"
 #include "dev_cell.hpp"
 #include "capi_util.hpp"
@@ -43,11 +42,6 @@ constexpr double VSCALE = 1e-6;
 __device__ __forceinline__ float gelu(float z)
 {
   return 0.5f * z * (1.f + tanhf(C_GELU * (z + 0.044715f * z * z * z)));
-}
-__device__ __forceinline__ float gelu_grad(float z)
-{
-  float t = tanhf(C_GELU * (z + 0.044715f * z * z * z));
-  return 0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * C_GELU * (1.f + 3.f * 0.044715f * z * z);
 }
 
 // ---------------------------------------------------------------------------
@@ -189,111 +183,334 @@ __global__ void __launch_bounds__(256) k_u2p_guess(koral_params P, long n, const
 }
 
 // ---------------------------------------------------------------------------
-// FP32 training kernels; activations are [feature][sample] with stride B
+// FP32 training kernels.  A step of B samples is three launches: k_mlp_pass
+// (forward, loss, and backward to every layer's dZ), k_mlp_grad (weight and
+// bias gradients, summed over chunks of CHUNK samples) and k_mlp_reduce (the
+// chunks' sum in a fixed order, and the Adam update).  All products run on the
+// FP32 matrix cores (v_mfma_f32_16x16x4_f32: lane l holds A[l%16][l/16],
+// B[l/16][l%16] and D[4(l/16)..+3][l%16]; FP32 products and sums).  A step of
+// 4096 samples is 0.9 GFLOP, 6 us at the matrix cores' rate; with one thread
+// per output and a launch per layer it took 290 us (16 launches), most of it
+// re-reading operands.
 // ---------------------------------------------------------------------------
-// Z[o][b] = bias[o] + sum_i W[o][i] X[i][b];  A = gelu(Z) when act
-__global__ void __launch_bounds__(256) k_dense_fwd(const float *__restrict__ W, const float *__restrict__ bias,
-                                                   const float *__restrict__ X, int I, int O, int B,
-                                                   float *__restrict__ Z, float *__restrict__ A, int act)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int TILE = 16;    // samples of a k_mlp_pass block: 4096 samples give each CU one
+constexpr int CHUNK = 128;  // samples of a k_mlp_grad block
+constexpr int SMAX = BMAX / CHUNK;
+constexpr int HS = 20;      // LDS row stride of a [feature][TILE] activation tile: the four
+                            // quarters of a wave read rows 4 apart, 16 banks from each other
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
 {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x, o = blockIdx.y;
-  if (b >= B) return;
-  float z = bias[o];
-  for (int i = 0; i < I; i++) z += W[o * I + i] * X[i * B + b];
-  Z[o * B + b] = z;
-  if (A) A[o * B + b] = act ? gelu(z) : z;
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// loss = sum (Y - T)^2 / (4 B), dY = 2 (Y - T) / (4 B); one block
-__global__ void __launch_bounds__(256) k_mse(const float *__restrict__ Y, const float *__restrict__ T, int B,
-                                             float *__restrict__ dY, float *__restrict__ loss)
+// a = gelu(z) and its derivative from one tanh
+__device__ __forceinline__ void gelu_both(float z, float &a, float &d)
 {
-  __shared__ float red[256];
-  float s = 0.f;
-  const float scale = 1.f / (float)(NOUT * B);
-  for (int k = threadIdx.x; k < NOUT * B; k += blockDim.x) {
-    float r = Y[k] - T[k];
-    s += r * r;
-    dY[k] = 2.f * r * scale;
+  float t = tanhf(C_GELU * (z + 0.044715f * z * z * z));
+  a = 0.5f * z * (1.f + t);
+  d = 0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * C_GELU * (1.f + 3.f * 0.044715f * z * z);
+}
+
+// Two 16-row tiles of W h (W [128][128], rows o and o + 16 at this lane) added
+// to acc: lane quarter q takes inputs 16 j + 4 q + r, one 16-byte load each j
+__device__ __forceinline__ void dense_rows(const float *__restrict__ W, const float (*h)[HS], int o, int q, int b,
+                                           f32x4 acc[2])
+{
+#pragma unroll
+  for (int j = 0; j < NH / 16; j++) {
+    const f32x4 w0 = *(const f32x4 *)(W + o * NH + 16 * j + 4 * q);
+    const f32x4 w1 = *(const f32x4 *)(W + (o + 16) * NH + 16 * j + 4 * q);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float x = h[16 * j + 4 * q + r][b];
+      acc[0] = mfma4(w0[r], x, acc[0]);
+      acc[1] = mfma4(w1[r], x, acc[1]);
+    }
   }
-  red[threadIdx.x] = s;
+}
+// the same for W^T h: columns i and i + 16 of W
+__device__ __forceinline__ void dense_cols(const float *__restrict__ W, const float (*h)[HS], int i, int q, int b,
+                                           f32x4 acc[2])
+{
+#pragma unroll
+  for (int j = 0; j < NH / 16; j++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int o = 16 * j + 4 * q + r;
+      const float x = h[o][b];
+      acc[0] = mfma4(W[o * NH + i], x, acc[0]);
+      acc[1] = mfma4(W[o * NH + i + 16], x, acc[1]);
+    }
+}
+
+// activations and gradients of a training batch, [feature][sample] with
+// stride BMAX
+struct TrainBufs {
+  float *A[3], *dZ[3], *dY, *lpart;
+};
+
+// One block takes TILE samples through the whole network: wave w holds the
+// output rows 32 w..32 w + 31 of each hidden layer, the activations pass
+// through LDS, the weights come from L2.  TRAIN: the squared error, and the
+// backward pass; samples past B leave zeros.
+template <bool TRAIN>
+__global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, const float *__restrict__ X,
+                                                  const float *__restrict__ T, int B, float *__restrict__ Yout,
+                                                  TrainBufs tb)
+{
+  __shared__ float h[2][NH][HS];
+  __shared__ float part[4][NOUT][TILE];
+  __shared__ float dy[NOUT][TILE];
+  __shared__ float sq[NOUT * TILE];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+  const int b0 = blockIdx.x * TILE, bs = b0 + c;  // this lane's sample
+  const bool live = bs < B;
+  if (TRAIN && b0 >= B) {
+    for (int k = threadIdx.x; k < NH * TILE; k += 256) {
+      const long at = (long)(k / TILE) * BMAX + b0 + k % TILE;
+#pragma unroll
+      for (int l = 0; l < 3; l++) tb.A[l][at] = tb.dZ[l][at] = 0.f;
+    }
+    if (threadIdx.x < NOUT * TILE) tb.dY[(long)(threadIdx.x / TILE) * BMAX + b0 + threadIdx.x % TILE] = 0.f;
+    if (threadIdx.x == 0) tb.lpart[blockIdx.x] = 0.f;
+    return;
+  }
+  const int row = 32 * wave;
+  float gp[3][2][4];  // gelu' of this lane's rows of each hidden layer
+  f32x4 acc[2];
+  auto hidden = [&](int l, float (*dst)[HS]) {
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int o = row + 16 * t + 4 * q + r;
+        float a;
+        gelu_both(acc[t][r], a, gp[l][t][r]);
+        dst[o][c] = a;
+        if (TRAIN) tb.A[l][(long)o * BMAX + bs] = live ? a : 0.f;
+      }
+  };
+  auto bias = [&](int ob) {
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[t][r] = th[ob + row + 16 * t + 4 * q + r];
+  };
+  // layer 1: 11 inputs, the twelfth of the three K = 4 products is zero
+  bias(OB1);
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    const int k = 4 * j + q;
+    const float x = (k < NIN && live) ? X[(long)k * B + bs] : 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      acc[t] = mfma4(k < NIN ? th[OW1 + (row + 16 * t + c) * NIN + k] : 0.f, x, acc[t]);
+  }
+  hidden(0, h[0]);
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+  bias(OB2);
+  dense_rows(th + OW2, h[0], row + c, q, c, acc);
+  hidden(1, h[1]);
+  __syncthreads();
+  bias(OB3);
+  dense_rows(th + OW3, h[1], row + c, q, c, acc);
+  hidden(2, h[0]);
+  __syncthreads();
+  // output layer: each wave a quarter of the inputs
+  {
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int k = row + 16 * j + 4 * q + r;
+        y = mfma4(c < NOUT ? th[OW4 + c * NH + k] : 0.f, h[0][k][c], y);
+      }
+    if (q == 0)
+#pragma unroll
+      for (int r = 0; r < 4; r++) part[wave][r][c] = y[r];
   }
-  if (threadIdx.x == 0) *loss = red[0] * scale;
-}
-
-// dZ = dA * gelu'(Z)
-__global__ void __launch_bounds__(256) k_gelu_bwd(const float *__restrict__ dA, const float *__restrict__ Z, long n,
-                                                  float *__restrict__ dZ)
-{
-  long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) dZ[k] = dA[k] * gelu_grad(Z[k]);
-}
-
-// dX[i][b] = sum_o W[o][i] dZ[o][b]
-__global__ void __launch_bounds__(256) k_dense_bwd_x(const float *__restrict__ W, const float *__restrict__ dZ,
-                                                     int I, int O, int B, float *__restrict__ dX)
-{
-  const int b = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
-  if (b >= B) return;
-  float s = 0.f;
-  for (int o = 0; o < O; o++) s += W[o * I + i] * dZ[o * B + b];
-  dX[i * B + b] = s;
-}
-
-// gW[o][i] = sum_b dZ[o][b] X[i][b] for i < I, gb[o] = sum_b dZ[o][b]
-// (column i = I); block (o, 16 columns), fixed-order reduction
-__global__ void __launch_bounds__(256) k_dense_bwd_w(const float *__restrict__ dZ, const float *__restrict__ X,
-                                                     int I, int B, float *__restrict__ gW, float *__restrict__ gb)
-{
-  __shared__ float part[16][257];
-  const int o = blockIdx.x, i0 = blockIdx.y * 16, t = threadIdx.x;
-  float acc[16];
+  __syncthreads();
+  if (threadIdx.x < NOUT * TILE) {
+    const int o = threadIdx.x / TILE, b = threadIdx.x % TILE;
+    const float y = th[OB4 + o] + part[0][o][b] + part[1][o][b] + part[2][o][b] + part[3][o][b];
+    const bool in = b0 + b < B;
+    if (Yout && in) Yout[(long)o * B + b0 + b] = y;
+    if (TRAIN) {
+      const float r = in ? y - T[(long)o * B + b0 + b] : 0.f;
+      const float d = 2.f * r * (1.f / (float)(NOUT * B));
+      dy[o][b] = d;
+      sq[threadIdx.x] = r * r;
+      tb.dY[(long)o * BMAX + b0 + b] = d;
+    }
+  }
+  if (!TRAIN) return;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float s = 0.f;
+    for (int k = 0; k < NOUT * TILE; k++) s += sq[k];
+    tb.lpart[blockIdx.x] = s;
+  }
+  // dZ of a hidden layer from dA in acc
+  auto back = [&](int l, float (*dst)[HS]) {
 #pragma unroll
-  for (int j = 0; j < 16; j++) acc[j] = 0.f;
-  for (int b = t; b < B; b += 256) {
-    const float d = dZ[o * B + b];
+    for (int t = 0; t < 2; t++)
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-      const int i = i0 + j;
-      const float x = (i < I) ? X[i * B + b] : (i == I ? 1.f : 0.f);
-      acc[j] += d * x;
+      for (int r = 0; r < 4; r++) {
+        const int i = row + 16 * t + 4 * q + r;
+        const float d = acc[t][r] * gp[l][t][r];
+        dst[i][c] = d;
+        tb.dZ[l][(long)i * BMAX + bs] = live ? d : 0.f;
+      }
+  };
+#pragma unroll
+  for (int t = 0; t < 2; t++) acc[t] = mfma4(th[OW4 + q * NH + row + 16 * t + c], dy[q][c], f32x4{0.f, 0.f, 0.f, 0.f});
+  back(2, h[1]);
+  __syncthreads();
+  acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  dense_cols(th + OW3, h[1], row + c, q, c, acc);
+  back(1, h[0]);
+  __syncthreads();
+  acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  dense_cols(th + OW2, h[0], row + c, q, c, acc);
+  back(0, h[1]);
+}
+
+// Gradients over one chunk of samples, gpart[chunk][NPARAM]: blockIdx.y 0..3 the
+// halves (64 outputs) of layers 2 and 3, a wave 32 x 64 weights; 4 the first
+// and the last layer.
+__global__ void __launch_bounds__(256) k_mlp_grad(const float *__restrict__ X, int B, TrainBufs tb,
+                                                  float *__restrict__ gpart)
+{
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+  const int s0 = blockIdx.x * CHUNK;
+  float *g = gpart + (long)blockIdx.x * NPARAM;
+  // D tile of the weights W[rows][cols] at (o0, i0)
+  auto store = [&](int ow, int width, int o0, int i0, int rows, int cols, const f32x4 &d) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int o = o0 + 4 * q + r, i = i0 + c;
+      if (o < rows && i < cols) g[ow + o * width + i] = d[r];
+    }
+  };
+  // sum over the chunk of row o0 + c's gradients from the lanes' parts
+  auto store_bias = [&](int ob, int rows, float sum) {
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (q == 0 && c < rows) g[ob + c] = sum;
+  };
+  if (blockIdx.y < 4) {
+    const int l = blockIdx.y < 2 ? 1 : 2;
+    const float *dz = tb.dZ[l], *a = tb.A[l - 1];
+    const int o0 = 64 * (blockIdx.y & 1) + 32 * (wave >> 1), i0 = 64 * (wave & 1);
+    f32x4 acc[2][4];
+    float sum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int j = 0; j < CHUNK / 16; j++) {
+      const int b = s0 + 16 * j + 4 * q;
+      f32x4 x[2], y[4];
+#pragma unroll
+      for (int t = 0; t < 2; t++) x[t] = *(const f32x4 *)(dz + (long)(o0 + 16 * t + c) * BMAX + b);
+#pragma unroll
+      for (int u = 0; u < 4; u++) y[u] = *(const f32x4 *)(a + (long)(i0 + 16 * u + c) * BMAX + b);
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          sum[t] += x[t][r];
+#pragma unroll
+          for (int u = 0; u < 4; u++) acc[t][u] = mfma4(x[t][r], y[u][r], acc[t][u]);
+        }
+    }
+    const int ow = l == 1 ? OW2 : OW3, ob = l == 1 ? OB2 : OB3;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) store(ow, NH, o0 + 16 * t, i0 + 16 * u, NH, NH, acc[t][u]);
+      if ((wave & 1) == 0) store_bias(ob + o0 + 16 * t, 16, sum[t]);
+    }
+    return;
+  }
+  f32x4 a1[2], a4[2];
+  float sum1[2] = {0.f, 0.f}, sum4 = 0.f;
+#pragma unroll
+  for (int t = 0; t < 2; t++) a1[t] = a4[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int w0 = 32 * wave;
+#pragma unroll 2
+  for (int j = 0; j < CHUNK / 16; j++) {
+    const int b = s0 + 16 * j + 4 * q;
+    f32x4 x1[2], y4[2], x4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      x1[t] = *(const f32x4 *)(tb.dZ[0] + (long)(w0 + 16 * t + c) * BMAX + b);
+      y4[t] = *(const f32x4 *)(tb.A[2] + (long)(w0 + 16 * t + c) * BMAX + b);
+    }
+    if (c < NOUT) x4 = *(const f32x4 *)(tb.dY + (long)c * BMAX + b);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float y1 = (c < NIN && b + r < B) ? X[(long)c * B + b + r] : 0.f;
+      sum4 += x4[r];
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        sum1[t] += x1[t][r];
+        a1[t] = mfma4(x1[t][r], y1, a1[t]);
+        a4[t] = mfma4(x4[r], y4[t][r], a4[t]);
+      }
     }
   }
 #pragma unroll
-  for (int j = 0; j < 16; j++) part[j][t] = acc[j];
-  __syncthreads();
-  if (t < 16) {
-    float s = 0.f;
-    for (int k = 0; k < 256; k++) s += part[t][k];
-    const int i = i0 + t;
-    if (i < I) gW[o * I + i] = s;
-    else if (i == I) gb[o] = s;
+  for (int t = 0; t < 2; t++) {
+    store(OW1, NIN, w0 + 16 * t, 0, NH, NIN, a1[t]);
+    store_bias(OB1 + w0 + 16 * t, 16, sum1[t]);
+    store(OW4, NH, 0, w0 + 16 * t, NOUT, NH, a4[t]);
   }
+  if (wave == 0) store_bias(OB4, NOUT, sum4);
 }
 
-__global__ void __launch_bounds__(256) k_adam(float *__restrict__ th, const float *__restrict__ g,
-                                              float *__restrict__ m, float *__restrict__ v, int n, float lr,
-                                              float b1, float b2, float c1, float c2, float eps)
+// g = the chunks' sum; adam: the Adam update of th.  The last block
+// sums the loss over the nb blocks of k_mlp_pass.
+__global__ void __launch_bounds__(256) k_mlp_reduce(float *__restrict__ th, const float *__restrict__ gpart, int chunks,
+                                                    float *__restrict__ g, float *__restrict__ m,
+                                                    float *__restrict__ v, bool adam, float lr, float b1, float b2,
+                                                    float c1, float c2, float eps, const float *__restrict__ lpart,
+                                                    int nb, int B, float *__restrict__ loss)
 {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  float gk = g[k];
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ float red[256];
+    red[threadIdx.x] = (int)threadIdx.x < nb ? lpart[threadIdx.x] : 0.f;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = red[0] * (1.f / (float)(NOUT * B));
+    return;
+  }
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= NPARAM) return;
+  float gk = 0.f;
+  for (int q = 0; q < chunks; q++) gk += gpart[(long)q * NPARAM + k];
+  g[k] = gk;
+  if (!adam) return;
   float mk = b1 * m[k] + (1.f - b1) * gk;
   float vk = b2 * v[k] + (1.f - b2) * gk * gk;
   m[k] = mk;
   v[k] = vk;
   th[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
 }
+static_assert(BMAX / TILE <= 256, "k_mlp_reduce sums one loss part per thread");
+static_assert(BMAX % CHUNK == 0 && CHUNK % TILE == 0, "tiles fill chunks");
 
 // ---------------------------------------------------------------------------
 // BF16 matrix-core inference
 // ---------------------------------------------------------------------------
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ unsigned short f2bf(float x)
 {
@@ -302,41 +519,55 @@ __device__ __forceinline__ unsigned short f2bf(float x)
   return (unsigned short)(u >> 16);
 }
 
-// weights in BF16 as the matrix cores read them: W1 padded to 16 inputs,
-// W4 padded to 16 outputs (zero rows/columns)
+// Weights in BF16 in the order the matrix cores' lanes read them (see
+// k_mlp_infer): a fragment is a 16 x 16 block of W[out][in], lane l's four
+// values W[16 ot + l%16][16 kc + 4 (l/16)..+3] next to each other and the
+// lanes in order, so a wave reads a fragment as 512 consecutive bytes (rows
+// of W lie 256 bytes apart: 16 lanes would meet in the same LDS banks).  W1
+// is padded to 16 inputs, W4 to 16 outputs, with zeros.
+constexpr int FRAG = 256;  // values of a fragment
 constexpr int PW1 = 0, PW2 = PW1 + NH * 16, PW3 = PW2 + NH * NH, PW4 = PW3 + NH * NH, NPACK = PW4 + 16 * NH;
 
 __global__ void __launch_bounds__(256) k_pack_bf16(const float *__restrict__ th, unsigned short *__restrict__ wp)
 {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= NPACK) return;
+  // row and column of value k of its fragment
+  const int l = (k % FRAG) / 4, ro = l % 16, co = 4 * (l / 16) + k % 4;
   float v = 0.f;
   if (k < PW2) {
-    int o = (k - PW1) / 16, i = (k - PW1) % 16;
-    v = i < NIN ? th[OW1 + o * NIN + i] : 0.f;
-  } else if (k < PW3) {
-    v = th[OW2 + (k - PW2)];
+    const int o = 16 * ((k - PW1) / FRAG) + ro;
+    v = co < NIN ? th[OW1 + o * NIN + co] : 0.f;
   } else if (k < PW4) {
-    v = th[OW3 + (k - PW3)];
+    const int base = k < PW3 ? PW2 : PW3, f = (k - base) / FRAG;
+    v = th[(k < PW3 ? OW2 : OW3) + (16 * (f / 8) + ro) * NH + 16 * (f % 8) + co];
   } else {
-    int o = (k - PW4) / NH, i = (k - PW4) % NH;
-    v = o < NOUT ? th[OW4 + o * NH + i] : 0.f;
+    v = ro < NOUT ? th[OW4 + ro * NH + 16 * ((k - PW4) / FRAG) + co] : 0.f;
   }
   wp[k] = f2bf(v);
 }
 
-// One wave per 16 cells.  For D = A B on the 16x16x16 BF16 matrix core,
-// lane l holds A[l%16][4(l/16)..+3] and B[4(l/16)..+3][l%16] and receives
-// D[4(l/16)..+3][l%16].  A is the activation tile [cell][k] and B the
-// transposed weights, B[k][o] = W[o][k], so both are 4 consecutive k.
-__global__ void __launch_bounds__(256) k_mlp_infer(const unsigned short *__restrict__ wp,
-                                                   const float *__restrict__ th, const float *__restrict__ feat,
-                                                   long n, float *__restrict__ out)
+// Each wave takes CT tiles of 16 cells through the network.  For D = A B on
+// the 16x16x16 BF16 matrix core, lane l holds A[l%16][4(l/16)..+3] and
+// B[4(l/16)..+3][l%16] and receives D[4(l/16)..+3][l%16].  A is a block of
+// the weights [out][in], B the activations [in][cell], so D holds the outputs
+// of one cell per lane as four consecutive inputs of the next layer: exactly
+// its B operand, and the activations never leave the registers.  The weights
+// sit in LDS (74 KB: two blocks of eight waves a CU) and a fragment read
+// serves CT tiles.  Bound by the 384 tanh of a cell (FP32 VALU), not by the
+// products: 2^20 cells take 423 us (1645 us with activations through LDS and
+// conflicting weight reads; two tiles a wave 435 us at two waves per SIMD,
+// 902 us at four, spilling).
+constexpr int CT = 1;
+constexpr int INFER_WAVES = 8;
+__global__ void __launch_bounds__(64 * INFER_WAVES, 4) k_mlp_infer(const unsigned short *__restrict__ wp,
+                                                                   const float *__restrict__ th,
+                                                                   const float *__restrict__ feat, long n,
+                                                                   float *__restrict__ out)
 {
-  __shared__ unsigned short sw[NPACK];
-  __shared__ float sb[3 * NH + 16];
-  __shared__ unsigned short sh[4][2][16][NH + 4];  // per wave: two activation tiles, padded rows
-  for (int k = threadIdx.x; k < NPACK; k += blockDim.x) sw[k] = wp[k];
+  __shared__ __align__(16) unsigned short sw[NPACK];
+  __shared__ __align__(16) float sb[3 * NH + 16];
+  for (int k = threadIdx.x; k < NPACK / 8; k += blockDim.x) ((uint4 *)sw)[k] = ((const uint4 *)wp)[k];
   for (int k = threadIdx.x; k < 3 * NH + 16; k += blockDim.x) {
     float v = 0.f;
     if (k < NH) v = th[OB1 + k];
@@ -347,73 +578,79 @@ __global__ void __launch_bounds__(256) k_mlp_infer(const unsigned short *__restr
   }
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = lane & 15, kq = 4 * (lane >> 4);
-  for (long base = (long)blockIdx.x * 64; base < n; base += (long)gridDim.x * 64) {
-    const long c0 = base + 16 * wave;
-    // layer 1: A from the features (k < 11), zero padded
-    bf16x4 a;
-    {
-      const long c = c0 + row;
+  const int col = lane & 15, kq = 4 * (lane >> 4);
+  auto frag = [&](int base, int f) { return *(const bf16x4 *)&sw[base + f * FRAG + 4 * lane]; };
+  const long step = (long)gridDim.x * INFER_WAVES * 16 * CT;
+  for (long c0 = ((long)blockIdx.x * INFER_WAVES + wave) * 16 * CT; c0 < n; c0 += step) {
+    bf16x4 x[CT], h[CT][NH / 16];
+    // inputs: 11 features, zero padded
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
+      const long c = c0 + 16 * t + col;
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const int k = kq + q;
         const float v = (c < n && k < NIN) ? feat[k * n + c] : 0.f;
-        a[q] = (short)f2bf(v);
+        x[t][q] = (short)f2bf(v);
       }
     }
-    unsigned short(*h0)[NH + 4] = sh[wave][0];
-    unsigned short(*h1)[NH + 4] = sh[wave][1];
+    auto activate = [&](const f32x4 &acc, const float *bias, int ot) {
+      const f32x4 b = *(const f32x4 *)&bias[16 * ot + kq];
+      bf16x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[r] = (short)f2bf(gelu(acc[r] + b[r]));
+      return v;
+    };
 #pragma unroll
     for (int ot = 0; ot < NH / 16; ot++) {
-      const int o = 16 * ot + row;
-      bf16x4 b = *(const bf16x4 *)&sw[PW1 + o * 16 + kq];
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+      const bf16x4 w = frag(PW1, ot);
 #pragma unroll
-      for (int r = 0; r < 4; r++) h0[kq + r][o] = f2bf(gelu(acc[r] + sb[o]));
+      for (int t = 0; t < CT; t++) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w, x[t], acc, 0, 0, 0);
+        h[t][ot] = activate(acc, sb, ot);
+      }
     }
-    __syncthreads();
-    // layers 2 and 3: 128 -> 128
-#pragma unroll
+    // layers 2 and 3: one copy of the code (it holds 64 inlined tanh)
+#pragma unroll 1
     for (int layer = 0; layer < 2; layer++) {
-      const int pw = layer == 0 ? PW2 : PW3;
-      unsigned short(*hin)[NH + 4] = layer == 0 ? h0 : h1;
-      unsigned short(*hout)[NH + 4] = layer == 0 ? h1 : h0;
-      const float *bias = sb + (layer + 1) * NH;
+      bf16x4 hn[CT][NH / 16];
+      const int base = layer == 0 ? PW2 : PW3;
 #pragma unroll
       for (int ot = 0; ot < NH / 16; ot++) {
-        const int o = 16 * ot + row;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        // the weights of one row of fragments in flight at a time
+        compiler_fence();
+        f32x4 acc[CT];
+#pragma unroll
+        for (int t = 0; t < CT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kc = 0; kc < NH / 16; kc++) {
-          bf16x4 av = *(const bf16x4 *)&hin[row][16 * kc + kq];
-          bf16x4 bv = *(const bf16x4 *)&sw[pw + o * NH + 16 * kc + kq];
-          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+          const bf16x4 w = frag(base, 8 * ot + kc);
+#pragma unroll
+          for (int t = 0; t < CT; t++)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w, h[t][kc], acc[t], 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++) hout[kq + r][o] = f2bf(gelu(acc[r] + bias[o]));
+        for (int t = 0; t < CT; t++) hn[t][ot] = activate(acc[t], sb + (layer + 1) * NH, ot);
       }
-      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < CT; t++)
+#pragma unroll
+        for (int ot = 0; ot < NH / 16; ot++) h[t][ot] = hn[t][ot];
     }
     // output layer: 128 -> 4 (padded to 16)
-    {
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kc = 0; kc < NH / 16; kc++) {
-        bf16x4 av = *(const bf16x4 *)&h0[row][16 * kc + kq];
-        bf16x4 bv = *(const bf16x4 *)&sw[PW4 + row * NH + 16 * kc + kq];
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
-      }
-      const int o = row;
-      if (o < NOUT) {
+      for (int kc = 0; kc < NH / 16; kc++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(frag(PW4, kc), h[t][kc], acc, 0, 0, 0);
+      const long c = c0 + 16 * t + col;
+      if (kq == 0 && c < n) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const long c = c0 + kq + r;
-          if (c < n) out[o * n + c] = acc[r] + sb[3 * NH + o];
-        }
+        for (int o = 0; o < NOUT; o++) out[o * n + c] = acc[o] + sb[3 * NH + o];
       }
     }
-    __syncthreads();
   }
 }
 
@@ -464,21 +701,43 @@ struct koral_hip_mlp {
   unsigned short *wp = nullptr;
   bool packed = false;
   int step = 0;
-  float *Z[3] = {}, *A[3] = {}, *Y = nullptr, *dY = nullptr, *d0 = nullptr, *d1 = nullptr, *loss = nullptr;
-  std::vector<void *> allocs;
-  template <class T>
-  int alloc(T **p, size_t count)
+  TrainBufs tb{};
+  float *gpart = nullptr, *loss = nullptr;
+  void *mem = nullptr;  // one allocation holds them all
+  // f(ptr, count) for every device buffer
+  template <class F>
+  void buffers(F &&f)
   {
-    void *q = nullptr;
-    int rc = check_hip(hipMalloc(&q, count * sizeof(T)), "hipMalloc mlp");
+    f(th, (size_t)NPARAM);
+    f(this->m, (size_t)NPARAM);
+    f(v, (size_t)NPARAM);
+    f(g, (size_t)NPARAM);
+    f(norm, (size_t)NNORM);
+    f(wp, (size_t)NPACK);
+    for (int k = 0; k < 3; k++) f(tb.A[k], (size_t)NH * BMAX);
+    for (int k = 0; k < 3; k++) f(tb.dZ[k], (size_t)NH * BMAX);
+    f(tb.dY, (size_t)NOUT * BMAX);
+    f(tb.lpart, (size_t)(BMAX / TILE));
+    f(gpart, (size_t)SMAX * NPARAM);
+    f(loss, (size_t)1);
+  }
+  int alloc()
+  {
+    size_t bytes = 0;
+    auto padded = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    buffers([&](auto *&p, size_t n) { bytes += padded(n * sizeof(*p)); });
+    int rc = check_hip(hipMalloc(&mem, bytes), "hipMalloc mlp");
     if (rc) return rc;
-    allocs.push_back(q);
-    *p = (T *)q;
+    char *at = (char *)mem;
+    buffers([&](auto *&p, size_t n) {
+      p = (std::remove_reference_t<decltype(p)>)at;
+      at += padded(n * sizeof(*p));
+    });
     return 0;
   }
   ~koral_hip_mlp()
   {
-    for (void *q : allocs) (void)hipFree(q);
+    if (mem) (void)hipFree(mem);
   }
 };
 
@@ -493,36 +752,18 @@ int pack(koral_hip_mlp *m, hipStream_t s)
   return check_launch("mlp pack");
 }
 
-// forward pass of a batch X [11][B] into m->Z/A and m->Y [4][B]
-void forward(koral_hip_mlp *m, const float *X, int B, hipStream_t s)
+// loss and gradient of the mean squared error of a batch X [11][B] into
+// m->loss and m->g, and with adam the update of step m->step
+int train(koral_hip_mlp *m, const float *X, const float *T, int B, bool adam, float lr, hipStream_t s)
 {
-  dim3 gb((B + 255) / 256, NH);
-  k_dense_fwd<<<gb, 256, 0, s>>>(m->th + OW1, m->th + OB1, X, NIN, NH, B, m->Z[0], m->A[0], 1);
-  k_dense_fwd<<<gb, 256, 0, s>>>(m->th + OW2, m->th + OB2, m->A[0], NH, NH, B, m->Z[1], m->A[1], 1);
-  k_dense_fwd<<<gb, 256, 0, s>>>(m->th + OW3, m->th + OB3, m->A[1], NH, NH, B, m->Z[2], m->A[2], 1);
-  dim3 go((B + 255) / 256, NOUT);
-  k_dense_fwd<<<go, 256, 0, s>>>(m->th + OW4, m->th + OB4, m->A[2], NH, NOUT, B, m->Y, nullptr, 0);
-}
-
-// loss and gradient of the mean squared error into m->g
-void backward(koral_hip_mlp *m, const float *X, const float *T, int B, hipStream_t s)
-{
-  k_mse<<<1, 256, 0, s>>>(m->Y, T, B, m->dY, m->loss);
-  const long nh = (long)NH * B;
-  // output layer
-  k_dense_bwd_w<<<dim3(NOUT, (NH + 1 + 15) / 16), 256, 0, s>>>(m->dY, m->A[2], NH, B, m->g + OW4, m->g + OB4);
-  k_dense_bwd_x<<<dim3((B + 255) / 256, NH), 256, 0, s>>>(m->th + OW4, m->dY, NH, NOUT, B, m->d0);
-  k_gelu_bwd<<<grid1(nh), 256, 0, s>>>(m->d0, m->Z[2], nh, m->d1);
-  // layer 3
-  k_dense_bwd_w<<<dim3(NH, (NH + 1 + 15) / 16), 256, 0, s>>>(m->d1, m->A[1], NH, B, m->g + OW3, m->g + OB3);
-  k_dense_bwd_x<<<dim3((B + 255) / 256, NH), 256, 0, s>>>(m->th + OW3, m->d1, NH, NH, B, m->d0);
-  k_gelu_bwd<<<grid1(nh), 256, 0, s>>>(m->d0, m->Z[1], nh, m->d1);
-  // layer 2
-  k_dense_bwd_w<<<dim3(NH, (NH + 1 + 15) / 16), 256, 0, s>>>(m->d1, m->A[0], NH, B, m->g + OW2, m->g + OB2);
-  k_dense_bwd_x<<<dim3((B + 255) / 256, NH), 256, 0, s>>>(m->th + OW2, m->d1, NH, NH, B, m->d0);
-  k_gelu_bwd<<<grid1(nh), 256, 0, s>>>(m->d0, m->Z[0], nh, m->d1);
-  // layer 1
-  k_dense_bwd_w<<<dim3(NH, (NIN + 1 + 15) / 16), 256, 0, s>>>(m->d1, X, NIN, B, m->g + OW1, m->g + OB1);
+  const int chunks = (B + CHUNK - 1) / CHUNK, nb = chunks * (CHUNK / TILE);
+  const double b1 = 0.9, b2 = 0.999;
+  const float c1 = (float)(1. - pow(b1, m->step)), c2 = (float)(1. - pow(b2, m->step));
+  k_mlp_pass<true><<<nb, 256, 0, s>>>(m->th, X, T, B, nullptr, m->tb);
+  k_mlp_grad<<<dim3(chunks, 5), 256, 0, s>>>(X, B, m->tb, m->gpart);
+  k_mlp_reduce<<<(NPARAM + 255) / 256 + 1, 256, 0, s>>>(m->th, m->gpart, chunks, m->g, m->m, m->v, adam, lr, (float)b1,
+                                                        (float)b2, c1, c2, 1e-8f, m->tb.lpart, nb, B, m->loss);
+  return check_launch("mlp train");
 }
 
 int read_loss(koral_hip_mlp *m, float *loss, hipStream_t s)
@@ -543,18 +784,7 @@ int koral_hip_mlp_create(int kind, koral_hip_mlp **out)
   if (!out || kind < 0 || kind > 3) return set_error(KORAL_E_ARG, "mlp_create: bad arguments");
   auto *m = new koral_hip_mlp();
   m->kind = kind;
-  int rc = 0;
-  float **vecs[4] = {&m->th, &m->m, &m->v, &m->g};
-  for (int k = 0; k < 4 && !rc; k++) rc = m->alloc(vecs[k], NPARAM);
-  if (!rc) rc = m->alloc(&m->norm, NNORM);
-  if (!rc) rc = m->alloc(&m->wp, NPACK);
-  for (int k = 0; k < 3 && !rc; k++) rc = m->alloc(&m->Z[k], (size_t)NH * BMAX);
-  for (int k = 0; k < 3 && !rc; k++) rc = m->alloc(&m->A[k], (size_t)NH * BMAX);
-  if (!rc) rc = m->alloc(&m->Y, (size_t)NOUT * BMAX);
-  if (!rc) rc = m->alloc(&m->dY, (size_t)NOUT * BMAX);
-  if (!rc) rc = m->alloc(&m->d0, (size_t)NH * BMAX);
-  if (!rc) rc = m->alloc(&m->d1, (size_t)NH * BMAX);
-  if (!rc) rc = m->alloc(&m->loss, 1);
+  int rc = m->alloc();
   if (!rc) rc = check_hip(hipMemset(m->m, 0, NPARAM * sizeof(float)), "memset");
   if (!rc) rc = check_hip(hipMemset(m->v, 0, NPARAM * sizeof(float)), "memset");
   if (rc) {
@@ -668,9 +898,8 @@ int koral_hip_mlp_forward(koral_hip_mlp *m, const float *X, int B, float *Y, voi
 {
   if (!m || !X || !Y || B < 1 || B > BMAX) return set_error(KORAL_E_ARG, "mlp_forward: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  forward(m, X, B, s);
-  int rc = check_hip(hipMemcpyAsync(Y, m->Y, (size_t)NOUT * B * sizeof(float), hipMemcpyDeviceToDevice, s), "copy");
-  return rc ? rc : check_launch("mlp_forward");
+  k_mlp_pass<false><<<(B + TILE - 1) / TILE, 256, 0, s>>>(m->th, X, nullptr, B, Y, m->tb);
+  return check_launch("mlp_forward");
 }
 
 int koral_hip_mlp_grad(koral_hip_mlp *m, const float *X, const float *T, int B, float *grad, float *loss,
@@ -678,11 +907,9 @@ int koral_hip_mlp_grad(koral_hip_mlp *m, const float *X, const float *T, int B, 
 {
   if (!m || !X || !T || B < 1 || B > BMAX) return set_error(KORAL_E_ARG, "mlp_grad: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  forward(m, X, B, s);
-  backward(m, X, T, B, s);
-  int rc = grad ? check_hip(hipMemcpyAsync(grad, m->g, NPARAM * sizeof(float), hipMemcpyDeviceToDevice, s), "copy")
-                : 0;
-  if (!rc) rc = check_launch("mlp_grad");
+  int rc = train(m, X, T, B, false, 0.f, s);
+  if (!rc && grad)
+    rc = check_hip(hipMemcpyAsync(grad, m->g, NPARAM * sizeof(float), hipMemcpyDeviceToDevice, s), "copy");
   return rc ? rc : read_loss(m, loss, s);
 }
 
@@ -691,14 +918,9 @@ int koral_hip_mlp_train_step(koral_hip_mlp *m, const float *X, const float *T, i
 {
   if (!m || !X || !T || B < 1 || B > BMAX) return set_error(KORAL_E_ARG, "mlp_train_step: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  forward(m, X, B, s);
-  backward(m, X, T, B, s);
   m->step++;
-  const double b1 = 0.9, b2 = 0.999;
-  const float c1 = (float)(1. - pow(b1, m->step)), c2 = (float)(1. - pow(b2, m->step));
-  k_adam<<<grid1(NPARAM), 256, 0, s>>>(m->th, m->g, m->m, m->v, NPARAM, lr, (float)b1, (float)b2, c1, c2, 1e-8f);
+  int rc = train(m, X, T, B, true, lr, s);
   m->packed = false;
-  int rc = check_launch("mlp_train_step");
   return rc ? rc : read_loss(m, loss, s);
 }
 
@@ -709,9 +931,10 @@ int koral_hip_mlp_infer(koral_hip_mlp *m, const float *feat, long n, float *Y, v
   hipStream_t s = (hipStream_t)stream;
   int rc = pack(m, s);
   if (rc) return rc;
-  long blocks = (n + 63) / 64;
-  if (blocks > 2048) blocks = 2048;
-  k_mlp_infer<<<(unsigned)blocks, 256, 0, s>>>(m->wp, m->th, feat, n, Y);
+  const long per = 16L * CT * INFER_WAVES;
+  long blocks = (n + per - 1) / per;
+  if (blocks > 512) blocks = 512;
+  k_mlp_infer<<<(unsigned)blocks, 64 * INFER_WAVES, 0, s>>>(m->wp, m->th, feat, n, Y);
   return check_launch("mlp_infer");
 }
 
