@@ -758,19 +758,35 @@ KD_INL double ff_Rtt(const double *pp, const GT &g, double *ucon_out)
 // ---------------------------------------------------------------------------
 // high-level inversion and floors
 // ---------------------------------------------------------------------------
+// The hot inversion and, where it fails, the entropy inversion: one inlined
+// copy of the solver in a loop over the equation (four copies in a kernel's
+// full path made it 100 to 200 KB of code, several times the instruction
+// cache).  etype: the equation to start with, and on return the one that
+// ended it.
+template <int MAG, int RAD, bool WAVE, int WG, class GT>
+KD_INL int u2p_hot_entropy(const koral_params &P, const double *uu, double *pp, const GT &g, int &etype)
+{
+  int r;
+#pragma unroll 1
+  for (;; etype++) {
+    r = u2p_solver_W<MAG, RAD, WAVE, WG>(P, uu, pp, g, etype);
+    if (r >= 0 || etype == 1) return r;
+  }
+}
+
 // u2p, u2p.c:176-485 (type 0)
 // With DEFER a state whose hot inversion fails is left for a later pass:
 // the function returns U2P_DEFERRED at once and the caller redoes the state
 // with DEFER false, so the entropy inversion is not inlined into the common
 // path.  A failed hot inversion leaves pp as it was unless it failed with
 // -105 (negative density after the update), so such a redo may start at the
-// entropy inversion (SKIP_HOT) and reach the same state; U2P_DEFERRED_105
+// entropy inversion (skip_hot) and reach the same state; U2P_DEFERRED_105
 // marks the other cases, where the redo runs the hot inversion again: -105,
 // and a hot inversion stopped by the budget (DEFER only, see u2p_solver_W).
 constexpr int U2P_DEFERRED = 1, U2P_DEFERRED_105 = 2;
-template <int MAG, int RAD, bool DEFER = false, bool SKIP_HOT = false, bool WAVE = false, int WG = WAVE_GROUP>
+template <int MAG, int RAD, bool DEFER = false, bool WAVE = false, int WG = WAVE_GROUP>
 KD_FUN int u2p(const koral_params &P, const double *uu0, double *pp, const Geom &g, int *corrected, int *fixups,
-               int budget = 0)
+               int budget = 0, bool skip_hot = false)
 {
   constexpr int NV = Lay<MAG, RAD>::NV;
   double uu[NV], ppbak[NV];
@@ -789,12 +805,13 @@ KD_FUN int u2p(const koral_params &P, const double *uu0, double *pp, const Geom 
     uu[0] = P.rhofloor * gdetu;
     ret = -2;
   }
-  u2pret = SKIP_HOT ? -1 : u2p_solver_W<MAG, RAD, WAVE, WG>(P, uu, pp, g, 0, 0., nullptr, DEFER ? budget : 0);
-  if (u2pret < 0) {
-    if (DEFER) return (u2pret == -105 || u2pret == U2P_OVER_BUDGET) ? U2P_DEFERRED_105 : U2P_DEFERRED;
-    ret = -1;
-    u2pret = u2p_solver_W<MAG, RAD, WAVE, WG>(P, uu, pp, g, 1);
-    if (u2pret < 0) ret = -2;
+  if constexpr (DEFER) {
+    u2pret = u2p_solver_W<MAG, RAD, WAVE, WG>(P, uu, pp, g, 0, 0., nullptr, budget);
+    if (u2pret < 0) return (u2pret == -105 || u2pret == U2P_OVER_BUDGET) ? U2P_DEFERRED_105 : U2P_DEFERRED;
+  } else {
+    int etype = skip_hot ? 1 : 0;
+    u2pret = u2p_hot_entropy<MAG, RAD, WAVE, WG>(P, uu, pp, g, etype);
+    if (etype == 1) ret = -1;
   }
   if (u2pret < 0) {
     ret = -3;
@@ -864,8 +881,8 @@ KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g)
       p2u_mhd<MAG, RAD>(P, dpp, duu, g);
 #pragma unroll
       for (int i = 0; i < 9; i++) uu[i] += duu[i];
-      int rt = u2p_solver_W<MAG, RAD, WAVE, WG>(P, uu, pp, g, 0);
-      if (rt < 0) rt = u2p_solver_W<MAG, RAD, WAVE, WG>(P, uu, pp, g, 1);
+      int etype = 0;
+      (void)u2p_hot_entropy<MAG, RAD, WAVE, WG>(P, uu, pp, g, etype);
       ret = -1;
     }
   }
@@ -926,16 +943,16 @@ KD_FUN int floors_rad(const koral_params &P, double *pp, const Geom &g)
 // With DEFER a cell that needs the entropy inversion or the b^2/rho floor
 // returns CP_DEFERRED_HOT (its hot inversion failed and left pp as it was)
 // or CP_DEFERRED before writing uu (pp may be changed) and is redone by the
-// caller with DEFER false, with SKIP_HOT for CP_DEFERRED_HOT.
+// caller with DEFER false, with skip_hot for CP_DEFERRED_HOT.
 constexpr int CP_DEFERRED = 100, CP_DEFERRED_HOT = 101;
-template <int MAG, int RAD, bool DEFER = false, bool SKIP_HOT = false, bool WAVE = false, int WG = WAVE_GROUP>
+template <int MAG, int RAD, bool DEFER = false, bool WAVE = false, int WG = WAVE_GROUP>
 KD_FUN int calc_primitives(const koral_params &P, double *uu, double *pp, const Geom &g, int &fl_entr,
-                               int &fl_entr2, int &fl_hd, int &fl_rad, int budget = 0)
+                               int &fl_entr2, int &fl_hd, int &fl_rad, int budget = 0, bool skip_hot = false)
 {
   int corrected[3] = {0, 0, 0}, fixups[2] = {0, 0};
   fl_entr = 0;
   fl_entr2 = 0;
-  int r = u2p<MAG, RAD, DEFER, SKIP_HOT, WAVE, WG>(P, uu, pp, g, corrected, fixups, budget);
+  int r = u2p<MAG, RAD, DEFER, WAVE, WG>(P, uu, pp, g, corrected, fixups, budget, skip_hot);
   if (DEFER && r == U2P_DEFERRED) return CP_DEFERRED_HOT;
   if (DEFER && r == U2P_DEFERRED_105) return CP_DEFERRED;
   if (corrected[0] == 1) fl_entr = 1;

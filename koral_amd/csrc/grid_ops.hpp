@@ -1127,12 +1127,12 @@ struct OpU2P {
   // before the cell is left to the deferred pass (0: no bound); a cell with
   // a long run of W bumps or step halvings then runs them lane-parallel
   int budget = 0;
-  KD_INL Cnt3 operator()(long i) const { return cell<true, false, false>(i, list, cnt, true); }
+  KD_INL Cnt3 operator()(long i) const { return cell<true, false>(i, list, cnt, true, false); }
   // the deferring calc_primitives, or the full one (optionally from the
   // entropy inversion on) on cell i; WAVE: the calling wave's lanes all run
   // cell i together and only the lane with store writes it
-  template <bool DEFER, bool SKIP_HOT, bool WAVE, int WG = WAVE_GROUP>
-  KD_INL Cnt3 cell(long i, unsigned *lst, unsigned *len, bool store) const
+  template <bool DEFER, bool WAVE, int WG = WAVE_GROUP>
+  KD_INL Cnt3 cell(long i, unsigned *lst, unsigned *len, bool store, bool skip_hot) const
   {
     constexpr int NV = Lay<MAG, RAD>::NV;
     Box b{0, 0, 0, G.nx, G.ny, G.nz};
@@ -1145,7 +1145,7 @@ struct OpU2P {
     Geom g;
     geom_cell(G, ix, iy, g);
     int fe, fe2, fh, fr;
-    const int r = calc_primitives<MAG, RAD, DEFER, SKIP_HOT, WAVE, WG>(P, uu, pp, g, fe, fe2, fh, fr, DEFER ? budget : 0);
+    const int r = calc_primitives<MAG, RAD, DEFER, WAVE, WG>(P, uu, pp, g, fe, fe2, fh, fr, DEFER ? budget : 0, skip_hot);
     if (DEFER) {
       const bool defer = r == CP_DEFERRED || r == CP_DEFERRED_HOT;
       const long slot = append_index(defer, (unsigned)i, lst, len);
@@ -1185,8 +1185,7 @@ struct OpU2PFloor {
     const bool lead = WAVE ? t % WG == 0 : true;
     for (long j = WAVE ? t / WG : t; j < m; j += nw) {
       const long i = (long)op.list[j];
-      const Cnt3 c = op.why[j] ? op.template cell<false, true, WAVE, WG>(i, nullptr, nullptr, lead)
-                                : op.template cell<false, false, WAVE, WG>(i, nullptr, nullptr, lead);
+      const Cnt3 c = op.template cell<false, WAVE, WG>(i, nullptr, nullptr, lead, op.why[j] != 0);
 #pragma unroll
       for (int k = 0; k < 3; k++) sum.v[k] += c.v[k];
     }
