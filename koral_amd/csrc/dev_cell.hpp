@@ -186,20 +186,35 @@ KD_INL double Sfromu(const koral_params &P, double rho, double u)
   return rho * kd_log(kd_pow(gm1 * u, n) / kd_pow(rho, n + 1.0));
 }
 
+// Four-velocity and magnetic four-vector of a primitive state: functions of
+// its velocities and field alone, which the floors, the conserved state and
+// the fluxes of one state share
+struct MhdKin {
+  double ucon[4], ucov[4], bcon[4], bcov[4], bsq;
+};
+template <int MAG, class GT>
+KD_INL void mhd_kin(const double *pp, const GT &g, MhdKin &k)
+{
+  relr_to_4vel(pp[2], pp[3], pp[4], k.ucon, k.ucov, g);
+#pragma unroll
+  for (int i = 0; i < 4; i++) k.bcon[i] = k.bcov[i] = 0.;
+  k.bsq = 0.;
+  if (MAG) {
+    bcon4(pp[6], pp[7], pp[8], k.ucon, k.ucov, k.bcon);
+    lower(k.bcon, k.bcov, g);
+    k.bsq = dot4(k.bcon, k.bcov);
+  }
+}
+
 // p2u_mhd, p2u.c:56-159
 template <int MAG, int RAD, class GT>
-KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const GT &g)
+KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const GT &g, const MhdKin &k)
 {
+  const double *ucon = k.ucon, *ucov = k.ucov, *bcon = k.bcon, *bcov = k.bcov;
+  const double bsq = k.bsq;
   double gdetu = g.gdet;
   double rho = pp[0], u = pp[1];
-  double ucon[4], ucov[4], bcon[4] = {0., 0., 0., 0.}, bcov[4] = {0., 0., 0., 0.}, bsq = 0.;
   double S = pp[5];
-  relr_to_4vel(pp[2], pp[3], pp[4], ucon, ucov, g);
-  if (MAG) {
-    bcon4(pp[6], pp[7], pp[8], ucon, ucov, bcon);
-    lower(bcon, bcov, g);
-    bsq = dot4(bcon, bcov);
-  }
   double ut = ucon[0];
   double rhout = rho * ut;
   double Sut = S * ut;
@@ -224,6 +239,13 @@ KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const G
     uu[7] = gdetu * pp[7];
     uu[8] = gdetu * pp[8];
   }
+}
+template <int MAG, int RAD, class GT>
+KD_INL void p2u_mhd(const koral_params &P, const double *pp, double *uu, const GT &g)
+{
+  MhdKin k;
+  mhd_kin<MAG>(pp, g, k);
+  p2u_mhd<MAG, RAD>(P, pp, uu, g, k);
 }
 
 // p2u_rad (M1), p2u.c:253-307
@@ -835,13 +857,15 @@ KD_FUN int u2p(const koral_params &P, const double *uu0, double *pp, const Geom 
 // two inlined Newton inversions of that rare branch out of a kernel's
 // common path is what DEFER is for.
 constexpr int FLOORS_DEFERRED = 1;
+// kin: mhd_kin of the floored state.
 template <int MAG, int RAD, bool DEFER = false, bool WAVE = false, int WG = WAVE_GROUP>
-KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g)
+KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g, MhdKin &kin)
 {
   constexpr int NV = Lay<MAG, RAD>::NV;
   int ret = 0;
   double uu[NV];
-  if (MAG) p2u_mhd<MAG, RAD>(P, pp, uu, g);
+  mhd_kin<MAG>(pp, g, kin);
+  if (MAG && !DEFER) p2u_mhd<MAG, RAD>(P, pp, uu, g, kin);
   if (pp[0] < P.rhofloor) {
     pp[0] = P.rhofloor;
     ret = -1;
@@ -855,13 +879,9 @@ KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g)
     ret = -1;
   }
   if (MAG) {
-    double ucon[4], ucov[4], bcon[4], bcov[4];
-    relr_to_4vel(pp[2], pp[3], pp[4], ucon, ucov, g);
-    bcon4(pp[6], pp[7], pp[8], ucon, ucov, bcon);
-    lower(bcon, bcov, g);
-    double magpre = dot4(bcon, bcov) / 2.;
+    double magpre = kin.bsq / 2.;
     if (magpre > P.b2rhoratiomax * pp[0]) {
-      if (DEFER) return FLOORS_DEFERRED;
+      if constexpr (DEFER) return FLOORS_DEFERRED;
       double alp = 1. / sqrt(-g.G[0][0]);
       double ncov[4] = {-alp, 0., 0., 0.}, etacon[4];
       raise_(ncov, etacon, g);
@@ -883,6 +903,7 @@ KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g)
       for (int i = 0; i < 9; i++) uu[i] += duu[i];
       int etype = 0;
       (void)u2p_hot_entropy<MAG, RAD, WAVE, WG>(P, uu, pp, g, etype);
+      mhd_kin<MAG>(pp, g, kin);
       ret = -1;
     }
   }
@@ -900,6 +921,7 @@ KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g)
       pp[2] *= A;
       pp[3] *= A;
       pp[4] *= A;
+      mhd_kin<MAG>(pp, g, kin);
       ret = -1;
     }
   }
@@ -957,9 +979,11 @@ KD_FUN int calc_primitives(const koral_params &P, double *uu, double *pp, const 
   if (DEFER && r == U2P_DEFERRED_105) return CP_DEFERRED;
   if (corrected[0] == 1) fl_entr = 1;
   if (corrected[2] == 1) fl_entr2 = 1;
-  if (floors_mhd<MAG, RAD, DEFER, WAVE, WG>(P, pp, g) == FLOORS_DEFERRED && DEFER) return CP_DEFERRED;
+  MhdKin kin;
+  if (floors_mhd<MAG, RAD, DEFER, WAVE, WG>(P, pp, g, kin) == FLOORS_DEFERRED && DEFER) return CP_DEFERRED;
   if (RAD) floors_rad<MAG, RAD>(P, pp, g);
-  p2u<MAG, RAD>(P, pp, uu, g);
+  p2u_mhd<MAG, RAD>(P, pp, uu, g, kin);
+  if (RAD) p2u_rad<MAG, RAD>(pp, uu, g);
   fl_hd = (fixups[0] > 0) ? 1 : 0;
   fl_rad = (fixups[1] > 0) ? -1 : 0;
   return r;

@@ -541,20 +541,26 @@ struct OpReconRun {
   }
 };
 
-// Fluxes at the face (ix, iy, iz) of direction D from its floored face
-// states: physical fluxes, conserved states, HLL or LF with the wave speeds
-// of the two cells (f_calc_fluxes_at_faces finite.c:1297-1415)
+// Physical flux and conserved state of one side of a face, from its floored
+// state p and k = mhd_kin of it
+template <int MAG, int RAD, int D>
+KD_INL void face_side(const koral_params &P, const double *p, const Geom &g, const MhdKin &k, double *f, double *u)
+{
+  flux_prime<MAG, RAD>(P, p, D + 1, g, k, f);
+  p2u_mhd<MAG, RAD>(P, p, u, g, k);
+  if (RAD) p2u_rad<MAG, RAD>(p, u, g);
+}
+
+// HLL or LF at the face (ix, iy, iz) of direction D from the fluxes and
+// conserved states of its sides, with the wave speeds of the two cells
+// (f_calc_fluxes_at_faces finite.c:1297-1415)
 template <int MAG, int RAD, int D>
 KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
-                      int iy, int iz, const double *pL, const double *pR, const Geom &g, bool store = true)
+                      int iy, int iz, const double *fL, const double *uL, const double *fR, const double *uR,
+                      bool store = true)
 {
   constexpr int NV = Lay<MAG, RAD>::NV;
   constexpr int NVMHD = 6 + 3 * MAG;
-  double fL[NV], fR[NV], uL[NV], uR[NV];
-  flux_prime<MAG, RAD>(P, pL, D + 1, g, fL);
-  flux_prime<MAG, RAD>(P, pR, D + 1, g, fR);
-  kd::p2u<MAG, RAD>(P, pL, uL, g);
-  kd::p2u<MAG, RAD>(P, pR, uR, g);
   const long n = G.ncell;
   const long cR = cidx(G, ix, iy, iz), cL = cR - dir_stride<D>(G);
   const long f = fidx(G, D, ix, iy, iz);
@@ -578,6 +584,34 @@ KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__res
     }
     if (store) flb[iv * nf + f] = F;
   }
+}
+
+// The common path of a face from its two states: floors, fluxes, Riemann
+// solver, one side after the other (the four-vectors of a side serve its
+// floors, flux and conserved state and are gone before the other's).  Returns
+// true, with nothing stored, when a state needs the b^2/rho floor.
+template <int MAG, int RAD, int D>
+KD_INL bool face_common(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
+                        int iy, int iz, double *pL, double *pR, const Geom &g, unsigned i, unsigned *list,
+                        unsigned *cnt)
+{
+  constexpr int NV = Lay<MAG, RAD>::NV;
+  double fL[NV], uL[NV], fR[NV], uR[NV];
+  bool defer;
+  {
+    MhdKin k;
+    defer = floors_mhd<MAG, RAD, true>(P, pL, g, k) == FLOORS_DEFERRED;
+    face_side<MAG, RAD, D>(P, pL, g, k, fL, uL);
+  }
+  {
+    MhdKin k;
+    if (floors_mhd<MAG, RAD, true>(P, pR, g, k) == FLOORS_DEFERRED) defer = true;
+    face_side<MAG, RAD, D>(P, pR, g, k, fR, uR);
+  }
+  append_index(defer, i, list, cnt);
+  if (defer) return true;
+  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, fL, uL, fR, uR);
+  return false;
 }
 
 // face states of face i of a sweep box, stored by OpRecon
@@ -619,12 +653,7 @@ struct OpFlux {
     load_face_states<NV>(fs, b.size(), i, pL, pR);
     Geom g;
     geom_face(G, D, ix, iy, g);
-    const int dl = floors_mhd<MAG, RAD, true>(P, pL, g);
-    const int dr = floors_mhd<MAG, RAD, true>(P, pR, g);
-    const bool defer = dl == FLOORS_DEFERRED || dr == FLOORS_DEFERRED;
-    append_index(defer, (unsigned)i, list, cnt);
-    if (defer) return;
-    face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g);
+    face_common<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, (unsigned)i, list, cnt);
   }
 };
 
@@ -644,7 +673,8 @@ KD_INL void floors_pair(const koral_params &P, double *pL, double *pR, const Geo
     double ps[NV];
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) ps[iv] = right ? pR[iv] : pL[iv];
-    floors_mhd<MAG, RAD, false, true, 32>(P, ps, g);
+    MhdKin k;
+    floors_mhd<MAG, RAD, false, true, 32>(P, ps, g, k);
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) {
       pL[iv] = __shfl(ps[iv], lane & 31);
@@ -653,8 +683,35 @@ KD_INL void floors_pair(const koral_params &P, double *pL, double *pR, const Geo
     return;
   }
 #endif
-  floors_mhd<MAG, RAD, false, WAVE>(P, pL, g);
-  floors_mhd<MAG, RAD, false, WAVE>(P, pR, g);
+  MhdKin k;
+#pragma unroll 1
+  for (int side = 0; side < 2; side++) {
+    double ps[NV];
+#pragma unroll
+    for (int iv = 0; iv < NV; iv++) ps[iv] = side ? pR[iv] : pL[iv];
+    floors_mhd<MAG, RAD, false, WAVE>(P, ps, g, k);
+#pragma unroll
+    for (int iv = 0; iv < NV; iv++) {
+      pL[iv] = side ? pL[iv] : ps[iv];
+      pR[iv] = side ? ps[iv] : pR[iv];
+    }
+  }
+}
+
+// The rare path: the full floors on both states, then the same fluxes
+template <int MAG, int RAD, int D, bool WAVE>
+KD_INL void face_floored(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
+                         int iy, int iz, double *pL, double *pR, const Geom &g, bool store)
+{
+  constexpr int NV = Lay<MAG, RAD>::NV;
+  double fL[NV], uL[NV], fR[NV], uR[NV];
+  MhdKin k;
+  floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
+  mhd_kin<MAG>(pL, g, k);
+  face_side<MAG, RAD, D>(P, pL, g, k, fL, uL);
+  mhd_kin<MAG>(pR, g, k);
+  face_side<MAG, RAD, D>(P, pR, g, k, fR, uR);
+  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, fL, uL, fR, uR, store);
 }
 
 // The faces OpFlux left: the same face states, the full face floors, the
@@ -687,8 +744,7 @@ struct OpFluxFloor {
       load_face_states<NV>(fs, b.size(), i, pL, pR);
       Geom g;
       geom_face(G, D, ix, iy, g);
-      floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
-      face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
+      face_floored<MAG, RAD, D, WAVE>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
     }
   }
 };
@@ -741,12 +797,7 @@ struct OpSweep {
     face_states<MAG, RAD, ORDER, D>(P, G, p, ix, iy, iz, pL, pR);
     Geom g;
     geom_face(G, D, ix, iy, g);
-    const int dl = floors_mhd<MAG, RAD, true>(P, pL, g);
-    const int dr = floors_mhd<MAG, RAD, true>(P, pR, g);
-    const bool defer = dl == FLOORS_DEFERRED || dr == FLOORS_DEFERRED;
-    append_index(defer, (unsigned)i, list, cnt);
-    if (defer) return;
-    face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g);
+    face_common<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, (unsigned)i, list, cnt);
   }
 };
 
@@ -777,8 +828,7 @@ struct OpSweepFloor {
       face_states<MAG, RAD, ORDER, D>(P, G, p, ix, iy, iz, pL, pR);
       Geom g;
       geom_face(G, D, ix, iy, g);
-      floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
-      face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
+      face_floored<MAG, RAD, D, WAVE>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
     }
   }
 };
@@ -1367,6 +1417,26 @@ inline GridTune default_tune()
   t.u2p_group = 32;
   t.floor_nw = 4096;
   t.u2p_nw = 4096;
+  return t;
+}
+
+// The choices a new grid starts with.  On a magnetised grid with MP5 the
+// fused sweep saves the face states' round trip through HBM where the box is
+// large enough to fill the chip with its 168-register waves: 128x128x64 zones
+// 3.08 ms per step split, 2.78 fused in all directions; 39 600 zones are
+// faster with only the x2 sweep fused, 2-D ones too.  The other
+// reconstructions spill in the fused kernel.  The update's early loads
+// (update_pre) are never slower, 128x128x64 2.78 -> 2.68 ms, and 64-thread
+// blocks suit the face kernels, 2.68 -> 2.60 ms.
+inline GridTune grid_tune(const koral_params &P, const DGrid &G)
+{
+  GridTune t = default_tune();
+  if (P.mag && P.int_order == 4) {
+    const bool large = (long)G.nx * G.ny * G.nz >= 100000;
+    for (int d = 0; d < 3; d++) t.fused[d] = large || d == 1 ? 1 : 0;
+    t.block[K_FLUX] = 64;
+  }
+  t.update_pre = 1;
   return t;
 }
 

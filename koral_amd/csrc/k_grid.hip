@@ -523,10 +523,10 @@ int koral_hip_grid_create(const koral_params *P, const koral_grid_desc *D, koral
     return set_error(KORAL_E_ARG, "grid_create: missing metric tables");
   auto *g = new koral_hip_grid();
   GridBufs &s = g->b;
-  s.tune = default_tune();
   s.P = *P;
   DGrid &G = s.G;
   grid_layout(D, G);
+  s.tune = grid_tune(*P, G);
   const int nv = P->nv;
   int rc = 0;
   auto up = [&](const double *h, size_t n, const double **dst) {
