@@ -179,6 +179,10 @@ int koral_hip_mlp_grad(koral_hip_mlp *m, const float *X, const float *T, int B, 
 /* one Adam step (beta 0.9, 0.999, eps 1e-8) on the mean squared error */
 int koral_hip_mlp_train_step(koral_hip_mlp *m, const float *X, const float *T, int B, float lr, float *loss,
                              void *stream);
+/* koral_hip_mlp_train_step on the B samples idx[0..B-1] (device, each in [0, N)) of X [11][N]
+   and T [4][N]: a shuffled mini-batch without gathering it first.  idx NULL: all N = B. */
+int koral_hip_mlp_train_step_at(koral_hip_mlp *m, const float *X, const float *T, long N, const long *idx, int B,
+                                float lr, float *loss, void *stream);
 /* BF16 matrix-core inference: standardised outputs Y [4][n] */
 int koral_hip_mlp_infer(koral_hip_mlp *m, const float *feat, long n, float *Y, void *stream);
 /* Gate (kind 3) outputs Y applied to a gas start: gxg[i] (u of cell i) becomes NaN where the

@@ -41,7 +41,7 @@ def u2p(P, uu, pp, g20, G20):
     Returns (ret [n] int32, flags [7, n] int32)."""
     n = pp.shape[1]
     _chk(uu), _chk(pp), _chk(g20), _chk(G20)
-    ret = torch.zeros(n, dtype=torch.int32, device=pp.device)
+    ret = torch.empty(n, dtype=torch.int32, device=pp.device)  # written for every point
     flags = torch.zeros((7, n), dtype=torch.int32, device=pp.device)
     check(lib().koral_hip_u2p_batch(ctypes.byref(P), n, _ptr(uu), _ptr(pp), _ptr(g20), _ptr(G20), _ptr(ret),
                                     _ptr(flags), _stream()), "u2p")
@@ -78,7 +78,7 @@ def implicit(P, uu, pp, g20, G20, dt, global_time=0.0):
     Returns (flags [7, n], info [6, n]) int32 tensors."""
     n = pp.shape[1]
     flags = torch.zeros((7, n), dtype=torch.int32, device=pp.device)
-    info = torch.zeros((6, n), dtype=torch.int32, device=pp.device)
+    info = torch.empty((6, n), dtype=torch.int32, device=pp.device)  # written for every cell
     check(lib().koral_hip_implicit_batch(ctypes.byref(P), n, _ptr(_chk(uu)), _ptr(_chk(pp)), _ptr(_chk(g20)),
                                          _ptr(_chk(G20)), _ptr(_chk(dt)), float(global_time), _ptr(flags),
                                          _ptr(info), _stream()), "implicit")

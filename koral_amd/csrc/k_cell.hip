@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) k_p2u(koral_params P, long n, const doubl
 // result.  With both in one path the kernel took 364 registers, one wave per
 // SIMD.
 template <int MAG, int RAD>
-__global__ void __launch_bounds__(256, 2) k_u2p(koral_params P, long n, double *__restrict__ uu,
+__global__ void __launch_bounds__(256, RAD && MAG ? 1 : 2) k_u2p(koral_params P, long n, double *__restrict__ uu,
                                                 double *__restrict__ pp, const double *__restrict__ g20,
                                                 const double *__restrict__ G20, int *__restrict__ ret,
                                                 int *__restrict__ flags)

@@ -195,7 +195,7 @@ __global__ void __launch_bounds__(256) k_u2p_guess(koral_params P, long n, const
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int TILE = 16;    // samples of a k_mlp_pass block: 4096 samples give each CU one
-constexpr int CHUNK = 128;  // samples of a k_mlp_grad block
+constexpr int CHUNK = 64;   // samples of a k_mlp_grad block
 constexpr int SMAX = BMAX / CHUNK;
 constexpr int HS = 20;      // LDS row stride of a [feature][TILE] activation tile: the four
                             // quarters of a wave read rows 4 apart, 16 banks from each other
@@ -213,35 +213,38 @@ __device__ __forceinline__ void gelu_both(float z, float &a, float &d)
   d = 0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * C_GELU * (1.f + 3.f * 0.044715f * z * z);
 }
 
-// Two 16-row tiles of W h (W [128][128], rows o and o + 16 at this lane) added
-// to acc: lane quarter q takes inputs 16 j + 4 q + r, one 16-byte load each j
-__device__ __forceinline__ void dense_rows(const float *__restrict__ W, const float (*h)[HS], int o, int q, int b,
-                                           f32x4 acc[2])
+// A lane's weights of two 16-row tiles of W h (W [128][128], rows o and
+// o + 16): lane quarter q takes inputs 16 j + 4 q + r, one 16-byte load each j.
+// They are loaded a layer ahead, so that no layer waits for them.
+struct RowsW {
+  f32x4 w[2][NH / 16];
+};
+__device__ __forceinline__ void load_rows(const float *__restrict__ W, int o, int q, RowsW &k)
 {
 #pragma unroll
-  for (int j = 0; j < NH / 16; j++) {
-    const f32x4 w0 = *(const f32x4 *)(W + o * NH + 16 * j + 4 * q);
-    const f32x4 w1 = *(const f32x4 *)(W + (o + 16) * NH + 16 * j + 4 * q);
+  for (int j = 0; j < NH / 16; j++)
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const float x = h[16 * j + 4 * q + r][b];
-      acc[0] = mfma4(w0[r], x, acc[0]);
-      acc[1] = mfma4(w1[r], x, acc[1]);
-    }
-  }
+    for (int t = 0; t < 2; t++) k.w[t][j] = *(const f32x4 *)(W + (o + 16 * t) * NH + 16 * j + 4 * q);
 }
-// the same for W^T h: columns i and i + 16 of W
-__device__ __forceinline__ void dense_cols(const float *__restrict__ W, const float (*h)[HS], int i, int q, int b,
-                                           f32x4 acc[2])
+// the same of W^T h: columns i and i + 16 of W
+__device__ __forceinline__ void load_cols(const float *__restrict__ W, int i, int q, RowsW &k)
+{
+#pragma unroll
+  for (int j = 0; j < NH / 16; j++)
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int t = 0; t < 2; t++) k.w[t][j][r] = W[(16 * j + 4 * q + r) * NH + i + 16 * t];
+}
+__device__ __forceinline__ void dense(const RowsW &k, const float (*h)[HS], int q, int b, f32x4 acc[2])
 {
 #pragma unroll
   for (int j = 0; j < NH / 16; j++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int o = 16 * j + 4 * q + r;
-      const float x = h[o][b];
-      acc[0] = mfma4(W[o * NH + i], x, acc[0]);
-      acc[1] = mfma4(W[o * NH + i + 16], x, acc[1]);
+      const float x = h[16 * j + 4 * q + r][b];
+      acc[0] = mfma4(k.w[0][j][r], x, acc[0]);
+      acc[1] = mfma4(k.w[1][j][r], x, acc[1]);
     }
 }
 
@@ -251,14 +254,24 @@ struct TrainBufs {
   float *A[3], *dZ[3], *dY, *lpart;
 };
 
+// A batch of B samples: column b of the batch is column idx[b] of X [11][N] and
+// T [4][N], or column b itself without idx (N = B then).  A training loop over
+// shuffled samples passes the permutation and keeps its pairs in place: the
+// kernels gather the 60 bytes of a sample themselves.
+struct Batch {
+  const float *X, *T;
+  long N;
+  const long *idx;
+  __device__ __forceinline__ long col(int b) const { return idx ? idx[b] : (long)b; }
+};
+
 // One block takes TILE samples through the whole network: wave w holds the
 // output rows 32 w..32 w + 31 of each hidden layer, the activations pass
 // through LDS, the weights come from L2.  TRAIN: the squared error, and the
 // backward pass; samples past B leave zeros.
 template <bool TRAIN>
-__global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, const float *__restrict__ X,
-                                                  const float *__restrict__ T, int B, float *__restrict__ Yout,
-                                                  TrainBufs tb)
+__global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, Batch bt, int B,
+                                                  float *__restrict__ Yout, TrainBufs tb)
 {
   __shared__ float h[2][NH][HS];
   __shared__ float part[4][NOUT][TILE];
@@ -267,6 +280,7 @@ __global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
   const int b0 = blockIdx.x * TILE, bs = b0 + c;  // this lane's sample
   const bool live = bs < B;
+  const long xc = live ? bt.col(bs) : 0;
   if (TRAIN && b0 >= B) {
     for (int k = threadIdx.x; k < NH * TILE; k += 256) {
       const long at = (long)(k / TILE) * BMAX + b0 + k % TILE;
@@ -298,25 +312,30 @@ __global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, 
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[t][r] = th[ob + row + 16 * t + 4 * q + r];
   };
+  RowsW wa, wb;
+  load_rows(th + OW2, row + c, q, wa);
   // layer 1: 11 inputs, the twelfth of the three K = 4 products is zero
   bias(OB1);
 #pragma unroll
   for (int j = 0; j < 3; j++) {
     const int k = 4 * j + q;
-    const float x = (k < NIN && live) ? X[(long)k * B + bs] : 0.f;
+    const float x = (k < NIN && live) ? bt.X[k * bt.N + xc] : 0.f;
 #pragma unroll
     for (int t = 0; t < 2; t++)
       acc[t] = mfma4(k < NIN ? th[OW1 + (row + 16 * t + c) * NIN + k] : 0.f, x, acc[t]);
   }
   hidden(0, h[0]);
+  load_rows(th + OW3, row + c, q, wb);
   __syncthreads();
   bias(OB2);
-  dense_rows(th + OW2, h[0], row + c, q, c, acc);
+  dense(wa, h[0], q, c, acc);
   hidden(1, h[1]);
+  if (TRAIN) load_cols(th + OW3, row + c, q, wa);
   __syncthreads();
   bias(OB3);
-  dense_rows(th + OW3, h[1], row + c, q, c, acc);
+  dense(wb, h[1], q, c, acc);
   hidden(2, h[0]);
+  if (TRAIN) load_cols(th + OW2, row + c, q, wb);
   __syncthreads();
   // output layer: each wave a quarter of the inputs
   {
@@ -339,7 +358,7 @@ __global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, 
     const bool in = b0 + b < B;
     if (Yout && in) Yout[(long)o * B + b0 + b] = y;
     if (TRAIN) {
-      const float r = in ? y - T[(long)o * B + b0 + b] : 0.f;
+      const float r = in ? y - bt.T[o * bt.N + bt.col(b0 + b)] : 0.f;
       const float d = 2.f * r * (1.f / (float)(NOUT * B));
       dy[o][b] = d;
       sq[threadIdx.x] = r * r;
@@ -370,19 +389,18 @@ __global__ void __launch_bounds__(256) k_mlp_pass(const float *__restrict__ th, 
   back(2, h[1]);
   __syncthreads();
   acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  dense_cols(th + OW3, h[1], row + c, q, c, acc);
+  dense(wa, h[1], q, c, acc);
   back(1, h[0]);
   __syncthreads();
   acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  dense_cols(th + OW2, h[0], row + c, q, c, acc);
+  dense(wb, h[0], q, c, acc);
   back(0, h[1]);
 }
 
 // Gradients over one chunk of samples, gpart[chunk][NPARAM]: blockIdx.y 0..3 the
 // halves (64 outputs) of layers 2 and 3, a wave 32 x 64 weights; 4 the first
 // and the last layer.
-__global__ void __launch_bounds__(256) k_mlp_grad(const float *__restrict__ X, int B, TrainBufs tb,
-                                                  float *__restrict__ gpart)
+__global__ void __launch_bounds__(256, 1) k_mlp_grad(Batch bt, int B, TrainBufs tb, float *__restrict__ gpart)
 {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
   const int s0 = blockIdx.x * CHUNK;
@@ -411,7 +429,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float *__restrict__ X, i
     for (int t = 0; t < 2; t++)
 #pragma unroll
       for (int u = 0; u < 4; u++) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
+#pragma unroll
     for (int j = 0; j < CHUNK / 16; j++) {
       const int b = s0 + 16 * j + 4 * q;
       f32x4 x[2], y[4];
@@ -442,7 +460,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float *__restrict__ X, i
 #pragma unroll
   for (int t = 0; t < 2; t++) a1[t] = a4[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int w0 = 32 * wave;
-#pragma unroll 2
+#pragma unroll
   for (int j = 0; j < CHUNK / 16; j++) {
     const int b = s0 + 16 * j + 4 * q;
     f32x4 x1[2], y4[2], x4 = {0.f, 0.f, 0.f, 0.f};
@@ -454,7 +472,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float *__restrict__ X, i
     if (c < NOUT) x4 = *(const f32x4 *)(tb.dY + (long)c * BMAX + b);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const float y1 = (c < NIN && b + r < B) ? X[(long)c * B + b + r] : 0.f;
+      const float y1 = (c < NIN && b + r < B) ? bt.X[c * bt.N + bt.col(b + r)] : 0.f;
       sum4 += x4[r];
 #pragma unroll
       for (int t = 0; t < 2; t++) {
@@ -495,6 +513,7 @@ __global__ void __launch_bounds__(256) k_mlp_reduce(float *__restrict__ th, cons
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= NPARAM) return;
   float gk = 0.f;
+#pragma unroll 8
   for (int q = 0; q < chunks; q++) gk += gpart[(long)q * NPARAM + k];
   g[k] = gk;
   if (!adam) return;
@@ -752,15 +771,15 @@ int pack(koral_hip_mlp *m, hipStream_t s)
   return check_launch("mlp pack");
 }
 
-// loss and gradient of the mean squared error of a batch X [11][B] into
-// m->loss and m->g, and with adam the update of step m->step
-int train(koral_hip_mlp *m, const float *X, const float *T, int B, bool adam, float lr, hipStream_t s)
+// loss and gradient of the mean squared error of a batch into m->loss and
+// m->g, and with adam the update of step m->step
+int train(koral_hip_mlp *m, const Batch &bt, int B, bool adam, float lr, hipStream_t s)
 {
   const int chunks = (B + CHUNK - 1) / CHUNK, nb = chunks * (CHUNK / TILE);
   const double b1 = 0.9, b2 = 0.999;
   const float c1 = (float)(1. - pow(b1, m->step)), c2 = (float)(1. - pow(b2, m->step));
-  k_mlp_pass<true><<<nb, 256, 0, s>>>(m->th, X, T, B, nullptr, m->tb);
-  k_mlp_grad<<<dim3(chunks, 5), 256, 0, s>>>(X, B, m->tb, m->gpart);
+  k_mlp_pass<true><<<nb, 256, 0, s>>>(m->th, bt, B, nullptr, m->tb);
+  k_mlp_grad<<<dim3(chunks, 5), 256, 0, s>>>(bt, B, m->tb, m->gpart);
   k_mlp_reduce<<<(NPARAM + 255) / 256 + 1, 256, 0, s>>>(m->th, m->gpart, chunks, m->g, m->m, m->v, adam, lr, (float)b1,
                                                         (float)b2, c1, c2, 1e-8f, m->tb.lpart, nb, B, m->loss);
   return check_launch("mlp train");
@@ -898,7 +917,7 @@ int koral_hip_mlp_forward(koral_hip_mlp *m, const float *X, int B, float *Y, voi
 {
   if (!m || !X || !Y || B < 1 || B > BMAX) return set_error(KORAL_E_ARG, "mlp_forward: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  k_mlp_pass<false><<<(B + TILE - 1) / TILE, 256, 0, s>>>(m->th, X, nullptr, B, Y, m->tb);
+  k_mlp_pass<false><<<(B + TILE - 1) / TILE, 256, 0, s>>>(m->th, Batch{X, nullptr, B, nullptr}, B, Y, m->tb);
   return check_launch("mlp_forward");
 }
 
@@ -907,7 +926,7 @@ int koral_hip_mlp_grad(koral_hip_mlp *m, const float *X, const float *T, int B, 
 {
   if (!m || !X || !T || B < 1 || B > BMAX) return set_error(KORAL_E_ARG, "mlp_grad: bad arguments");
   hipStream_t s = (hipStream_t)stream;
-  int rc = train(m, X, T, B, false, 0.f, s);
+  int rc = train(m, Batch{X, T, B, nullptr}, B, false, 0.f, s);
   if (!rc && grad)
     rc = check_hip(hipMemcpyAsync(grad, m->g, NPARAM * sizeof(float), hipMemcpyDeviceToDevice, s), "copy");
   return rc ? rc : read_loss(m, loss, s);
@@ -916,10 +935,17 @@ int koral_hip_mlp_grad(koral_hip_mlp *m, const float *X, const float *T, int B, 
 int koral_hip_mlp_train_step(koral_hip_mlp *m, const float *X, const float *T, int B, float lr, float *loss,
                              void *stream)
 {
-  if (!m || !X || !T || B < 1 || B > BMAX) return set_error(KORAL_E_ARG, "mlp_train_step: bad arguments");
+  return koral_hip_mlp_train_step_at(m, X, T, B, nullptr, B, lr, loss, stream);
+}
+
+int koral_hip_mlp_train_step_at(koral_hip_mlp *m, const float *X, const float *T, long N, const long *idx, int B,
+                                float lr, float *loss, void *stream)
+{
+  if (!m || !X || !T || B < 1 || B > BMAX || N < 1 || (!idx && N != B))
+    return set_error(KORAL_E_ARG, "mlp_train_step: bad arguments");
   hipStream_t s = (hipStream_t)stream;
   m->step++;
-  int rc = train(m, X, T, B, true, lr, s);
+  int rc = train(m, Batch{X, T, N, idx}, B, true, lr, s);
   m->packed = false;
   return rc ? rc : read_loss(m, loss, s);
 }

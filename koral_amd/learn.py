@@ -45,6 +45,7 @@ def _sig(L):
         "koral_hip_mlp_forward": [vp, vp, i, vp, vp],
         "koral_hip_mlp_grad": [vp, vp, vp, i, vp, vp, vp],
         "koral_hip_mlp_train_step": [vp, vp, vp, i, f, vp, vp],
+        "koral_hip_mlp_train_step_at": [vp, vp, vp, l, vp, i, f, vp, vp],
         "koral_hip_mlp_infer": [vp, vp, l, vp, vp],
         "koral_hip_mlp_guess": [vp, l, i, vp, vp, vp, vp],
         "koral_hip_implicit_batch_learned": [vp, vp, vp, l, vp, vp, vp, vp, vp, ctypes.c_double, i, vp, vp,
@@ -152,19 +153,25 @@ class Net:
         X [11][N], T [4][N] (device).  Returns the mean loss of each epoch
         (from every 64th batch)."""
         N = X.shape[1]
+        if X.shape[0] < NIN or T.shape[0] < NOUT or T.shape[1] < N:
+            raise ValueError("expected X [%d][N] and T [%d][N]" % (NIN, NOUT))
+        X, T = _chk(X.contiguous(), torch.float32), _chk(T[:, :N].contiguous(), torch.float32)
         gen = torch.Generator(device=X.device)
         gen.manual_seed(seed)
         hist = []
         for ep in range(epochs):
             perm = torch.randperm(N, device=X.device, generator=gen)
             losses = []
+            # the kernels take each mini-batch through the permutation: a
+            # gathered copy per batch cost as much as the training step
+            loss = ctypes.c_float(0.)
             for k, b0 in enumerate(range(0, N - batch + 1, batch)):
-                idx = perm[b0:b0 + batch]
-                xb = X[:, idx].contiguous()
-                tb = T[:, idx].contiguous()
-                l = self.step(xb, tb, lr, want_loss=(k % 64 == 0))
-                if l is not None:
-                    losses.append(l)
+                want = k % 64 == 0
+                check(self.L.koral_hip_mlp_train_step_at(
+                    self.h, _ptr(X), _ptr(T), N, ctypes.c_void_p(perm.data_ptr() + 8 * b0), batch, float(lr),
+                    ctypes.byref(loss) if want else None, _stream()), "mlp_train_step")
+                if want:
+                    losses.append(loss.value)
             hist.append(float(np.mean(losses)) if losses else float("nan"))
         return hist
 

@@ -1,5 +1,5 @@
 """The network kernels at the edges of their tiles: training batches around
-the 16-sample blocks and 128-sample gradient chunks (against the float64
+the 16-sample blocks and 64-sample gradient chunks (against the float64
 reference, with the tolerances of the whole-batch test: FP32 sums of up to 4096
 products), and inference batches around the 16-cell tiles and 128-cell blocks
 (a cell's outputs do not depend on the batch it is in)."""
@@ -17,7 +17,7 @@ def _net(seed):
     return M, th, Net(theta=th)
 
 
-@pytest.mark.parametrize("B", [1, 15, 16, 17, 127, 128, 129, 2051, 4095, 4096])
+@pytest.mark.parametrize("B", [1, 15, 16, 17, 63, 64, 65, 129, 2051, 4095, 4096])
 def test_training_batches(oracle, B):
     import torch
     M, th, net = _net(B)
@@ -45,3 +45,25 @@ def test_inference_batches(oracle):
     Y = net.infer(F)
     for n in (1, 15, 16, 17, 127, 128, 129, 65536, 70001):
         assert torch.equal(net.infer(F[:, :n].contiguous()), Y[:, :n]), n
+
+
+@pytest.mark.parametrize("B", [1, 130, 1000])
+def test_indexed_batches(oracle, B):
+    """fit takes its mini-batches through the permutation: the same steps as
+    on gathered copies, bit for bit."""
+    import torch
+    M, th, net = _net(9)
+    from koral_amd.learn import Net
+    other = Net(theta=th)
+    N = 3 * B + B // 2
+    g = torch.Generator("cuda").manual_seed(B)
+    X = torch.randn((M.NIN, N), device="cuda", generator=g)
+    T = torch.randn((M.NOUT, N), device="cuda", generator=g)
+    net.fit(X, T, epochs=2, lr=1e-3, batch=B, seed=4)
+    gen = torch.Generator("cuda").manual_seed(4)
+    for _ in range(2):
+        perm = torch.randperm(N, device="cuda", generator=gen)
+        for b0 in range(0, N - B + 1, B):
+            idx = perm[b0:b0 + B]
+            other.step(X[:, idx].contiguous(), T[:, idx].contiguous(), lr=1e-3)
+    assert np.array_equal(net.get()[0], other.get()[0])
