@@ -929,6 +929,13 @@ KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g, MhdKin &
   return ret;
 }
 
+template <int MAG, int RAD, bool DEFER = false, bool WAVE = false, int WG = WAVE_GROUP>
+KD_FUN int floors_mhd(const koral_params &P, double *pp, const Geom &g)
+{
+  MhdKin kin;
+  return floors_mhd<MAG, RAD, DEFER, WAVE, WG>(P, pp, g, kin);
+}
+
 // check_floors_rad, u2prad.c:687-800
 template <int MAG, int RAD>
 KD_FUN int floors_rad(const koral_params &P, double *pp, const Geom &g)

@@ -586,6 +586,21 @@ KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__res
   }
 }
 
+// the same from the floored states
+template <int MAG, int RAD, int D>
+KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
+                      int iy, int iz, const double *pL, const double *pR, const Geom &g, bool store = true)
+{
+  constexpr int NV = Lay<MAG, RAD>::NV;
+  double fL[NV], uL[NV], fR[NV], uR[NV];
+  MhdKin k;
+  mhd_kin<MAG>(pL, g, k);
+  face_side<MAG, RAD, D>(P, pL, g, k, fL, uL);
+  mhd_kin<MAG>(pR, g, k);
+  face_side<MAG, RAD, D>(P, pR, g, k, fR, uR);
+  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, fL, uL, fR, uR, store);
+}
+
 // The common path of a face from its two states: floors, fluxes, Riemann
 // solver, one side after the other (the four-vectors of a side serve its
 // floors, flux and conserved state and are gone before the other's).  Returns
@@ -673,8 +688,7 @@ KD_INL void floors_pair(const koral_params &P, double *pL, double *pR, const Geo
     double ps[NV];
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) ps[iv] = right ? pR[iv] : pL[iv];
-    MhdKin k;
-    floors_mhd<MAG, RAD, false, true, 32>(P, ps, g, k);
+    floors_mhd<MAG, RAD, false, true, 32>(P, ps, g);
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) {
       pL[iv] = __shfl(ps[iv], lane & 31);
@@ -683,13 +697,12 @@ KD_INL void floors_pair(const koral_params &P, double *pL, double *pR, const Geo
     return;
   }
 #endif
-  MhdKin k;
 #pragma unroll 1
   for (int side = 0; side < 2; side++) {
     double ps[NV];
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) ps[iv] = side ? pR[iv] : pL[iv];
-    floors_mhd<MAG, RAD, false, WAVE>(P, ps, g, k);
+    floors_mhd<MAG, RAD, false, WAVE>(P, ps, g);
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) {
       pL[iv] = side ? pL[iv] : ps[iv];
@@ -703,15 +716,8 @@ template <int MAG, int RAD, int D, bool WAVE>
 KD_INL void face_floored(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
                          int iy, int iz, double *pL, double *pR, const Geom &g, bool store)
 {
-  constexpr int NV = Lay<MAG, RAD>::NV;
-  double fL[NV], uL[NV], fR[NV], uR[NV];
-  MhdKin k;
   floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
-  mhd_kin<MAG>(pL, g, k);
-  face_side<MAG, RAD, D>(P, pL, g, k, fL, uL);
-  mhd_kin<MAG>(pR, g, k);
-  face_side<MAG, RAD, D>(P, pR, g, k, fR, uR);
-  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, fL, uL, fR, uR, store);
+  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, store);
 }
 
 // The faces OpFlux left: the same face states, the full face floors, the
@@ -1024,8 +1030,9 @@ struct OpCombSeq {
   // not overlap).  The sum a x + b y + c z is accumulated left to right,
   // the same operations in the same order as var().  No statement refers
   // to the result of the last, so COMB_MAXST - 1 results are kept.
+  // The result of statement uq goes to ur.
   template <int NV>
-  KD_INL void cell_vars(long c, const double coef[COMB_MAXST][3]) const
+  KD_INL void cell_vars(long c, const double coef[COMB_MAXST][3], int uq = -1, double *ur = nullptr) const
   {
     const unsigned cb = soa_off(c);
     double r[COMB_MAXST - 1][NV];
@@ -1062,6 +1069,9 @@ struct OpCombSeq {
       if (q < COMB_MAXST - 1)
 #pragma unroll
         for (int iv = 0; iv < NV; iv++) r[q][iv] = w[iv];
+      if (q == uq)
+#pragma unroll
+        for (int iv = 0; iv < NV; iv++) ur[iv] = w[iv];
     }
   }
   KD_INL void operator()(long i) const
@@ -1181,8 +1191,9 @@ struct OpU2P {
   // the deferring calc_primitives, or the full one (optionally from the
   // entropy inversion on) on cell i; WAVE: the calling wave's lanes all run
   // cell i together and only the lane with store writes it
-  template <bool DEFER, bool WAVE, int WG = WAVE_GROUP>
-  KD_INL Cnt3 cell(long i, unsigned *lst, unsigned *len, bool store, bool skip_hot) const
+  // GIVEN: the cell's u is given instead of read, and stored for a deferred cell
+  template <bool DEFER, bool WAVE, int WG = WAVE_GROUP, bool GIVEN = false>
+  KD_INL Cnt3 cell(long i, unsigned *lst, unsigned *len, bool store, bool skip_hot, const double *ug = nullptr) const
   {
     constexpr int NV = Lay<MAG, RAD>::NV;
     Box b{0, 0, 0, G.nx, G.ny, G.nz};
@@ -1191,7 +1202,12 @@ struct OpU2P {
     long c = cidx(G, ix, iy, iz);
     double pp[NV], uu[NV];
     load_p<MAG, RAD>(p, G.ncell, c, pp);
-    load_p<MAG, RAD>(u, G.ncell, c, uu);
+    if constexpr (GIVEN) {
+#pragma unroll
+      for (int iv = 0; iv < NV; iv++) uu[iv] = ug[iv];
+    } else {
+      load_p<MAG, RAD>(u, G.ncell, c, uu);
+    }
     Geom g;
     geom_cell(G, ix, iy, g);
     int fe, fe2, fh, fr;
@@ -1201,6 +1217,7 @@ struct OpU2P {
       const long slot = append_index(defer, (unsigned)i, lst, len);
       if (defer) {
         why[slot] = r == CP_DEFERRED_HOT ? 1 : 0;
+        if (GIVEN) store_p<MAG, RAD>(u, G.ncell, c, uu);
         return Cnt3{{0, 0, 0}};
       }
     }
@@ -1213,6 +1230,33 @@ struct OpU2P {
     fl[F_HDFIXUP * n + c] = (signed char)fh;
     fl[F_RADFIXUP * n + c] = (signed char)fr;
     return Cnt3{{fh != 0, fr != 0, fe != 0}};
+  }
+};
+
+// The stage algebra that forms u, and the common u2p pass on it, in one
+// launch: u is neither written by the one nor read by the other (a quarter of
+// the algebra's traffic, and a launch).  uq is the statement whose result is
+// the new u.  The first items clear the counters the
+// launches after this one append to (seq.zero).
+// 128x128x64: the algebra and the common u2p passes of a step 0.81 -> 0.73 ms.
+template <int MAG, int RAD>
+struct OpSeqU2P {
+  static constexpr int kind = K_U2P;
+  static constexpr int waves_per_simd = 2;
+  static constexpr int NV = Lay<MAG, RAD>::NV;
+  OpU2P<MAG, RAD> op;
+  OpCombSeq seq;
+  int uq;
+  KD_HD long size() const { return op.size(); }
+  KD_INL Cnt3 operator()(long i) const
+  {
+    const DGrid &G = op.G;
+    if (i < seq.nzero) seq.zero[i] = 0u;
+    const int ix = (int)(i % G.nx), iy = (int)((i / G.nx) % G.ny), iz = (int)(i / ((long)G.nx * G.ny));
+    double coef[COMB_MAXST][3], uu[NV] = {};
+    seq.coefs(coef);
+    seq.template cell_vars<NV>(cidx(G, ix, iy, iz), coef, uq, uu);
+    return op.template cell<true, false, WAVE_GROUP, true>(i, op.list, op.cnt, true, false, uu);
   }
 };
 
@@ -1449,12 +1493,12 @@ struct GridBufs {
   double *ws, *flb[3], *emf;
   double *fs[3];      // face states of the sweep of each direction, 2 NV x face_states_cap(G)
   unsigned *flist[3];  // faces of each sweep left to the b^2/rho floor pass, face_states_cap(G)
-  unsigned *fcnt;      // their counts [3], then the count of ulist
+  unsigned *fcnt;      // their counts [3], then two counts of ulist (step_rk2imex alternates them)
   unsigned *ulist;     // cells left to the full calc_primitives pass, nx ny nz
   unsigned char *uwhy;  // per ulist entry: the redo may skip the failed hot inversion
   double *pn, *un;
   int *mark;
-  double *ut0, *ut1, *uforget, *dut1, *dut2, *drt1, *drt2;
+  double *ut0, *ut1, *uforget, *dut1, *dut2, *drt1, *drt2;  // (dut2 is not stored: step_rk2imex)
   double *tsd;    // time-step density max (one double)
   double *clock;  // {t, dt} of the operators (device scalars)
   int *counters;  // step counters [6]
@@ -1492,7 +1536,7 @@ void grid_buffers(GridBufs &s, F &&f)
       f(s.fs[d], 2 * nv * face_states_cap(G), d == 0 ? "face states x" : d == 1 ? "face states y" : "face states z");
       f(s.flist[d], face_states_cap(G), d == 0 ? "floor list x" : d == 1 ? "floor list y" : "floor list z");
     }
-  f(s.fcnt, 4L, "list counts");
+  f(s.fcnt, 5L, "list counts");
   f(s.ulist, nd, "u2p list");
   f(s.uwhy, nd, "u2p list kinds");
   f(s.emf, 3L * (G.nx + 1) * (G.ny + 1) * (G.nz + 1), "emf");
@@ -1701,16 +1745,24 @@ void fixup(Ex &ex, const GridBufs &s, int type)
   });
 }
 
-// calc_u2p with its cell_fixup passes and the ghost refresh
+// calc_u2p with its cell_fixup passes and the ghost refresh.  seq: the stage
+// algebra that forms u first (statement uq's result), in the launch of the
+// common pass.  cnt: the counter of the deferred list; cleared says that an
+// earlier launch cleared it (seq clears others, see step_rk2imex).
 template <class Ex>
-void u2p(Ex &ex, const GridBufs &s, bool count_cleared = false)
+void u2p(Ex &ex, const GridBufs &s, bool cleared = false, const OpCombSeq *seq = nullptr, int uq = -1,
+         unsigned *cnt = nullptr)
 {
+  if (!cnt) cnt = s.fcnt + 3;
   dispatch(s.P, [&](auto t) {
     using T = decltype(t);
-    if (!count_cleared) ex.each(OpZeroU32{s.fcnt + 3, 1});
-    KD_CHECK(!count_cleared || s.fcnt[3] == 0u, "u2p: cell-list count not cleared", s.fcnt[3], 0, 0);
-    const OpU2P<T::MAG, T::RAD> op{s.P, s.G, s.u, s.p, s.fl, s.ulist, s.fcnt + 3, s.uwhy, s.tune.u2p_budget};
-    ex.count(op, s.counters + 3);
+    if (!cleared) ex.each(OpZeroU32{cnt, 1});
+    KD_CHECK(!cleared || *cnt == 0u, "u2p: cell-list count not cleared", *cnt, 0, 0);
+    const OpU2P<T::MAG, T::RAD> op{s.P, s.G, s.u, s.p, s.fl, s.ulist, cnt, s.uwhy, s.tune.u2p_budget};
+    if (seq)
+      ex.count(OpSeqU2P<T::MAG, T::RAD>{op, *seq, uq}, s.counters + 3);
+    else
+      ex.count(op, s.counters + 3);
     if (s.tune.floor_wave)
       if (s.tune.u2p_group == 32)
         ex.count(OpU2PFloor<T::MAG, T::RAD, true, 32>{op, s.tune.u2p_nw}, s.counters + 3);
@@ -1820,14 +1872,15 @@ void each_comb(Ex &ex, const GridBufs &s, const OpCombSeq &op)
   });
 }
 
+// out = a x in every interior cell; also clears one counter
 template <class Ex>
-void comb(Ex &ex, const GridBufs &s, double gamma, double *out, Coef a, const double *x,
-          Coef b = {Coef::CONST, 0.}, const double *y = nullptr, Coef c = {Coef::CONST, 0.},
-          const double *z = nullptr)
+void comb(Ex &ex, const GridBufs &s, double gamma, double *out, Coef a, const double *x, unsigned *zero)
 {
-  const int nt = z ? 3 : (y ? 2 : 1);
+  const CombTerm none{{Coef::CONST, 0.}, nullptr, 0};
   OpCombSeq op{s.G, s.P.nv, 1, {}, s.clock, gamma};
-  op.st[0] = CombStmt{out, nt, {CombTerm{a, x, 0}, CombTerm{b, y, 0}, CombTerm{c, z, 0}}};
+  op.st[0] = CombStmt{out, 1, {CombTerm{a, x, 0}, none, none}};
+  op.zero = zero;
+  op.nzero = 1;
   each_comb(ex, s, op);
 }
 
@@ -1845,76 +1898,86 @@ void step_rk2imex(Ex &ex, const GridBufs &s)
   auto A = [](Coef c, const double *x) { return CombTerm{c, x, 0}; };
   auto R = [](Coef c, int q) { return CombTerm{c, nullptr, q}; };
   const CombTerm none{{Coef::CONST, 0.}, nullptr, 0};
-  // each seq() precedes a u2p and also clears the four list counters of the
-  // u2p and of the explicit operator that follows it (no reader of them runs
-  // in between: the floor passes of the previous sweeps were joined)
-  // the statements of one launch (at most COMB_MAXST)
-  auto make = [&](std::initializer_list<CombStmt> l) {
+  // Each stage's algebra precedes a u2p.  The deferred lists' counters (faces
+  // 0..2, cells 3 and 4) are cleared without a launch of their own.  Fused
+  // (OpSeqU2P): the first and third u2p of a step count in 4 and clear 0..3 for
+  // the explicit operator and the u2p that follow; the second and fourth count
+  // in 3, and the second clears 4 for the third (the step's first launch clears
+  // it for the first).  The readers of a cleared counter are done: the u2p's redo pass by stream order,
+  // the floor passes by the joins.  Separate (comb_nv 0, or a grid of fewer than
+  // four cells): the algebra launch clears 0..3, every u2p counts in 3.
+  bool first = true;  // the first u2p of a pair
+  auto u2p_after = [&](std::initializer_list<CombStmt> l, int uq, double *uout) {
+    // the statements of one launch (at most COMB_MAXST)
     OpCombSeq op{s.G, s.P.nv, (int)l.size(), {}, s.clock, gamma};
     int q = 0;
     for (const CombStmt &st : l) op.st[q++] = st;
-    if (op.size() >= 4) {
+    const bool small = op.size() < 4;
+    if (s.tune.comb_nv && !small) {
+      op.zero = first ? s.fcnt : s.fcnt + 4;
+      op.nzero = first ? 4 : 1;
+      u2p(ex, s, true, &op, uq, s.fcnt + (first ? 4 : 3));
+    } else {
+      if (uout) op.st[uq].out = uout;
       op.zero = s.fcnt;
-      op.nzero = 4;
+      op.nzero = small ? 0 : 4;
+      if (small) ex.each(OpZeroU32{s.fcnt, 4});
+      each_comb(ex, s, op);
+      u2p(ex, s, true);
     }
-    return op;
+    first = !first;
+    do_correct(ex, s);
   };
-  auto seq = [&](std::initializer_list<CombStmt> l) {
-    const OpCombSeq op = make(l);
-    if (op.nzero == 0) ex.each(OpZeroU32{s.fcnt, 4});
-    each_comb(ex, s, op);
-  };
-  auto explicit_then = [&](std::initializer_list<CombStmt> l) {
-    // u2p ended with set_bc; without a polar correction p and u are unchanged
-    explicit_op(ex, s, !polar_correction_active(s), true);
-    seq(l);
-  };
+  // u2p ended with set_bc; without a polar correction p and u are unchanged
+  auto explicit_stage = [&] { explicit_op(ex, s, !polar_correction_active(s), true); };
   // Without radiation implicit_op is empty, so u does not change between
   // the first copies: ut1 = u = ut0 (1 u, the same bits), and drt1 =
   // (u - ut0) / (gamma dt) = idtg ut0 + midtg ut0, which the launches that
   // read drt1 recompute from ut0 with the same operations instead of
   // storing it.  Neither ut1 (first stage) nor drt1 is then stored or read.
+  // dut2 is read by its own launch alone and never stored.
   const bool norad = !s.P.rad;
   if (norad) {
-    seq({CombStmt{s.ut0, 1, {A(one, s.u), none, none}}});
+    ex.each(OpZeroU32{s.fcnt + 4, 1});
+    u2p_after({CombStmt{s.ut0, 1, {A(one, s.u), none, none}}}, 0, nullptr);
   } else {
-    comb(ex, s, gamma, s.ut0, one, s.u);
+    comb(ex, s, gamma, s.ut0, one, s.u, s.fcnt + 4);
     implicit_op(ex, s, gamma);
     // drt1 = (u - ut0) / (gamma dt); ut1 = u
-    seq({CombStmt{s.drt1, 2, {A(idtg, s.u), A(midtg, s.ut0), none}}, CombStmt{s.ut1, 1, {A(one, s.u), none, none}}});
+    u2p_after({CombStmt{s.drt1, 2, {A(idtg, s.u), A(midtg, s.ut0), none}}, CombStmt{s.ut1, 1, {A(one, s.u), none, none}}},
+              1, nullptr);
   }
-  u2p(ex, s, true);
-  do_correct(ex, s);
   // explicit; dut1 = (u - ut1) / dt; u = ut0 + dt dut1 + (1 - 2 gamma) dt drt1; uforget = u
+  explicit_stage();
   if (norad)
-    explicit_then({CombStmt{nullptr, 2, {A(idtg, s.ut0), A(midtg, s.ut0), none}},
-                   CombStmt{s.dut1, 2, {A(idt, s.u), A(midt, s.ut0), none}},
-                   CombStmt{s.u, 3, {A(one, s.ut0), R(dt1, 1), R(dtc, 0)}},
-                   CombStmt{s.uforget, 1, {R(one, 2), none, none}}});
+    u2p_after({CombStmt{nullptr, 2, {A(idtg, s.ut0), A(midtg, s.ut0), none}},
+               CombStmt{s.dut1, 2, {A(idt, s.u), A(midt, s.ut0), none}},
+               CombStmt{nullptr, 3, {A(one, s.ut0), R(dt1, 1), R(dtc, 0)}},
+               CombStmt{s.uforget, 1, {R(one, 2), none, none}}},
+              2, s.u);
   else
-    explicit_then({CombStmt{s.dut1, 2, {A(idt, s.u), A(midt, s.ut1), none}},
-                   CombStmt{s.u, 3, {A(one, s.ut0), R(dt1, 0), A(dtc, s.drt1)}},
-                   CombStmt{s.uforget, 1, {R(one, 1), none, none}}});
-  u2p(ex, s, true);
-  do_correct(ex, s);
+    u2p_after({CombStmt{s.dut1, 2, {A(idt, s.u), A(midt, s.ut1), none}},
+               CombStmt{nullptr, 3, {A(one, s.ut0), R(dt1, 0), A(dtc, s.drt1)}},
+               CombStmt{s.uforget, 1, {R(one, 1), none, none}}},
+              1, s.u);
   implicit_op(ex, s, gamma);
   // drt2 = (u - uforget) / (gamma dt); ut2 = u
-  seq({CombStmt{s.drt2, 2, {A(idtg, s.u), A(midtg, s.uforget), none}},
-       CombStmt{s.ut1, 1, {A(one, s.u), none, none}}});
-  u2p(ex, s, true);
-  do_correct(ex, s);
+  u2p_after({CombStmt{s.drt2, 2, {A(idtg, s.u), A(midtg, s.uforget), none}},
+             CombStmt{s.ut1, 1, {A(one, s.u), none, none}}},
+            1, nullptr);
   // explicit; dut2 = (u - ut2) / dt; u = ut0 + dt/2 (dut1 + dut2); u = u + dt/2 (drt1 + drt2)
+  explicit_stage();
   if (norad)
-    explicit_then({CombStmt{nullptr, 2, {A(idtg, s.ut0), A(midtg, s.ut0), none}},
-                   CombStmt{s.dut2, 2, {A(idt, s.u), A(midt, s.ut1), none}},
-                   CombStmt{nullptr, 3, {A(one, s.ut0), A(dth, s.dut1), R(dth, 1)}},
-                   CombStmt{s.u, 3, {R(one, 2), R(dth, 0), A(dth, s.drt2)}}});
+    u2p_after({CombStmt{nullptr, 2, {A(idtg, s.ut0), A(midtg, s.ut0), none}},
+               CombStmt{nullptr, 2, {A(idt, s.u), A(midt, s.ut1), none}},
+               CombStmt{nullptr, 3, {A(one, s.ut0), A(dth, s.dut1), R(dth, 1)}},
+               CombStmt{nullptr, 3, {R(one, 2), R(dth, 0), A(dth, s.drt2)}}},
+              3, s.u);
   else
-    explicit_then({CombStmt{s.dut2, 2, {A(idt, s.u), A(midt, s.ut1), none}},
-                   CombStmt{nullptr, 3, {A(one, s.ut0), A(dth, s.dut1), R(dth, 0)}},
-                   CombStmt{s.u, 3, {R(one, 1), A(dth, s.drt1), A(dth, s.drt2)}}});
-  u2p(ex, s, true);
-  do_correct(ex, s);
+    u2p_after({CombStmt{nullptr, 2, {A(idt, s.u), A(midt, s.ut1), none}},
+               CombStmt{nullptr, 3, {A(one, s.ut0), A(dth, s.dut1), R(dth, 0)}},
+               CombStmt{nullptr, 3, {R(one, 1), A(dth, s.drt1), A(dth, s.drt2)}}},
+              2, s.u);
 }
 
 }  // namespace kd
