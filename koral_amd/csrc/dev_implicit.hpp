@@ -114,7 +114,8 @@ KD_INL int imp_eval(const koral_params &P, const ImpKind &k, int mode, double *p
     ret = u2p_rad<MAG, RAD>(P, uu, pp, g, corr);
     cret = corr > 0 ? (mode == IMP_FINAL ? -2 : -1) : ret;
   }
-  if (mode == IMP_FINAL || (mode == IMP_TRIAL && !imp_trial_residual(whichprim, whicheq))) return 0;
+  // (a wave evaluates the next iterate beside its columns anyway)
+  if (mode == IMP_FINAL || (mode == IMP_TRIAL && (WG > 0 || !imp_trial_residual(whichprim, whicheq)))) return 0;
   if (ret < -1) return -1;
 
   compiler_fence();

@@ -1107,7 +1107,7 @@ struct OpCombSeqN : OpCombSeq {
 // registers: 128 VGPRs for MHD, so still 4 waves per SIMD; 3 with
 // radiation); otherwise p is loaded for the metric source and u at the end.
 // The arithmetic of every term is the same either way.
-template <int MAG, int RAD, bool PRE = false>
+template <int MAG, int RAD, bool PRE = false, bool CT = false>
 struct OpUpdate {
   static constexpr int kind = K_UPDATE;
   static constexpr int waves_per_simd = RAD ? 3 : 4;
@@ -1117,6 +1117,7 @@ struct OpUpdate {
   double *u;
   Flx F;
   const double *clk;  // device clock {t, dt}
+  const double *emf = nullptr;  // CT: OpEmf's corner EMFs
   KD_HD long size() const { return (long)G.nx * G.ny * G.nz; }
   KD_INL void operator()(long i) const
   {
@@ -1141,11 +1142,47 @@ struct OpUpdate {
     if (G.nz > 1) { fzl = fzidx(G, ix, iy, iz); fzr = fzidx(G, ix, iy, iz + 1); }
     const unsigned bxl = soa_off(fxl), bxr = soa_off(fxr), byl = soa_off(fyl), byr = soa_off(fyr),
                    bzl = soa_off(fzl), bzr = soa_off(fzr);
+    // CT: a face's field fluxes are means of two EMFs (OpCtFaces' expressions)
+    double bx[2][3] = {}, by[2][3] = {}, bz[2][3] = {};  // [left, right][component]
+    if constexpr (MAG && CT) {
+      const long ne = (long)(G.nx + 1) * (G.ny + 1) * (G.nz + 1), sy = G.nx + 1, sz = sy * (G.ny + 1);
+      const long e0 = ix + iy * sy + iz * sz;
+      auto E = [&](int k, int dx_, int dy_, int dz_) {
+        return soa_ld(emf, (k - 1) * ne, soa_off(e0 + dx_ + dy_ * sy + dz_ * sz));
+      };
+      double e1[2][2], e2[2][2], e3[2][2];  // e1[dy][dz], e2[dx][dz], e3[dx][dy]
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+          e1[q][r] = E(1, 0, q, r);
+          e2[q][r] = E(2, q, 0, r);
+          e3[q][r] = E(3, q, r, 0);
+        }
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        bx[q][1] = 0.5 * (e3[q][0] + e3[q][1]);
+        bx[q][2] = -0.5 * (e2[q][0] + e2[q][1]);
+        by[q][0] = -0.5 * (e3[0][q] + e3[1][q]);
+        by[q][2] = 0.5 * (e1[q][0] + e1[q][1]);
+        bz[q][0] = 0.5 * (e2[0][q] + e2[1][q]);
+        bz[q][1] = -0.5 * (e1[0][q] + e1[1][q]);
+      }
+    }
 #pragma unroll
     for (int iv = 0; iv < NV; iv++) {
-      du[iv] = -(soa_ld(F.x, iv * F.nfx, bxr) - soa_ld(F.x, iv * F.nfx, bxl)) * dt / dx;
-      if (G.ny > 1) du[iv] = du[iv] - (soa_ld(F.y, iv * F.nfy, byr) - soa_ld(F.y, iv * F.nfy, byl)) * dt / dy;
-      if (G.nz > 1) du[iv] = du[iv] - (soa_ld(F.z, iv * F.nfz, bzr) - soa_ld(F.z, iv * F.nfz, bzl)) * dt / dz;
+      const bool ct = MAG && CT && iv >= 6 && iv <= 8;
+      const int k = ct ? iv - 6 : 0;
+      const double xr = ct ? bx[1][k] : soa_ld(F.x, iv * F.nfx, bxr), xl = ct ? bx[0][k] : soa_ld(F.x, iv * F.nfx, bxl);
+      du[iv] = -(xr - xl) * dt / dx;
+      if (G.ny > 1) {
+        const double yr = ct ? by[1][k] : soa_ld(F.y, iv * F.nfy, byr), yl = ct ? by[0][k] : soa_ld(F.y, iv * F.nfy, byl);
+        du[iv] = du[iv] - (yr - yl) * dt / dy;
+      }
+      if (G.nz > 1) {
+        const double zr = ct ? bz[1][k] : soa_ld(F.z, iv * F.nfz, bzr), zl = ct ? bz[0][k] : soa_ld(F.z, iv * F.nfz, bzl);
+        du[iv] = du[iv] - (zr - zl) * dt / dz;
+      }
     }
     compiler_fence();
     if (!PRE) load_p<MAG, RAD>(p, G.ncell, c, pp);
@@ -1717,17 +1754,25 @@ void explicit_op(Ex &ex, const GridBufs &s, bool ghosts_current = false, bool co
     for (int d = 0; d < 3; d++)
       if (n[d] > 1) ex.join(d);
   Flx F{s.flb[0], s.flb[1], s.flb[2], G.nfx, G.nfy, G.nfz};
-  if (P.mag) {
-    ex.each(OpEmf{G, F, s.emf});
-    ex.each(OpCtFaces{G, F, s.emf});
-  }
+  // The update forms the field fluxes from the EMFs itself; the flux arrays
+  // keep the Riemann solver's (ct_faces sets flux-CT's where they are asked for)
+  if (P.mag) ex.each(OpEmf{G, F, s.emf});
   dispatch(P, [&](auto t) {
     using T = decltype(t);
     if (s.tune.update_pre)
-      ex.each(OpUpdate<T::MAG, T::RAD, true>{P, G, s.p, s.u, F, s.clock});
+      ex.each(OpUpdate<T::MAG, T::RAD, true, true>{P, G, s.p, s.u, F, s.clock, s.emf});
     else
-      ex.each(OpUpdate<T::MAG, T::RAD, false>{P, G, s.p, s.u, F, s.clock});
+      ex.each(OpUpdate<T::MAG, T::RAD, false, true>{P, G, s.p, s.u, F, s.clock, s.emf});
   });
+}
+
+// the B fluxes after flux-CT of every face, from the last explicit operator's
+// EMFs
+template <class Ex>
+void ct_faces(Ex &ex, const GridBufs &s)
+{
+  const DGrid &G = s.G;
+  if (s.P.mag) ex.each(OpCtFaces{G, Flx{s.flb[0], s.flb[1], s.flb[2], G.nfx, G.nfy, G.nfz}, s.emf});
 }
 
 template <class Ex>

@@ -558,6 +558,7 @@ int koral_hip_grid_create(const koral_params *P, const koral_grid_desc *D, koral
   for (int d = 0; d < 3 && !rc; d++)
     if (s.flb[d]) rc = check_hip(hipMemset(s.flb[d], 0, nv * (d == 0 ? G.nfx : d == 1 ? G.nfy : G.nfz) * sizeof(double)), "memset");
   if (!rc) rc = check_hip(hipMemset(s.ws, 0, NWS * nc * sizeof(double)), "memset");
+  if (!rc) rc = check_hip(hipMemset(s.emf, 0, 3L * (G.nx + 1) * (G.ny + 1) * (G.nz + 1) * sizeof(double)), "memset");
   if (rc) {
     delete g;
     return rc;
@@ -650,6 +651,10 @@ int koral_hip_grid_download_work(koral_hip_grid *g, int which, double *out)
   const double *src = which == 0 ? s.ws : s.flb[which - 1];
   if (!src) return set_error(KORAL_E_ARG, "grid_download_work: collapsed direction has no fluxes");
   long n = which == 0 ? (long)NWS * G.ncell : (long)s.P.nv * (which == 1 ? G.nfx : which == 2 ? G.nfy : G.nfz);
+  if (which > 0) {
+    HipExec ex = g->ex();
+    ct_faces(ex, s);
+  }
   int rc = check_hip(hipMemcpyAsync(out, src, n * sizeof(double), hipMemcpyDeviceToHost, g->s), "download work");
   return rc ? rc : check_hip(hipStreamSynchronize(g->s), "sync");
 }
