@@ -344,8 +344,9 @@ typedef struct koral_grid_tune {
   int fused[3];
   int floor_wave;
   int update_pre;   /* update kernel: 1 loads the cell's u and p with the fluxes */
-  int comb_nv;        /* 1: the stage-algebra kernel is compiled for the
-                         grid's variable count */
+  int comb_nv;        /* 1: the RK2IMEX stage algebra runs in the launch of
+                         the u2p that follows, compiled for the grid's
+                         variable count; 0: a launch of its own */
   int u2p_budget;     /* residual evaluations the common u2p pass spends on
                          a cell's hot inversion before leaving the cell to
                          the deferred (wave-parallel) pass; 0: no bound */

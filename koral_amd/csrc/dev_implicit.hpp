@@ -54,17 +54,19 @@ KD_INL int inverse44(const double *a, double *ia)
 
 enum { IMP_FAIL = -1, IMP_CONT = 0, IMP_OK = 1 };
 
-// One evaluation of an attempt's state machine: f_implicit and complete_state
-// as one function (rad.c:110-351, 880-950), so a solver that runs it in a loop holds a single inlined
-// copy.  mode EVAL: the residual f and its error at the state pp (pp is a work
-// copy); returns < 0 on failure as f_implicit.  TRIAL and FINAL: pp completed
-// as complete_state(final_pass = false / true) does, its return value in cret;
-// pp[5] is left alone (imp_finish sets it).  On the gas primitives with the
+// One evaluation of an attempt's state machine: the residual (rad.c:110-351)
+// and the completion of a state (rad.c:880-950) as one function, so a solver
+// that runs it in a loop holds a single inlined copy.  mode EVAL: the residual
+// f and its error at the state pp (pp is a work copy); returns < 0 where the
+// residual fails.  TRIAL and FINAL: pp completed as a damped trial / as the
+// converged state, the inversion's return value in cret; pp[5] is left alone (imp_finish sets it).  On the gas primitives with the
 // energy equation the residual at a completed state is the next iteration's:
 // both complete it with the same operations, so TRIAL evaluates it too
 // (imp_trial_residual).  pp0_u and Ehat0 = -ff_Rtt, of the old state, enter
 // the fluid-frame equation.  Template kind values < 0: the attempt's kind at
-// run time (k), the same in all lanes that run together.  WG as f_implicit.
+// run time (k), the same in all lanes that run together.  WG > 0: lanes of a
+// group that share the W inversion's trials (the wave-per-cell solve, whose
+// trials skip the residual: its next iterate is evaluated beside the columns).
 enum { IMP_EVAL = 0, IMP_TRIAL = 1, IMP_FINAL = 2 };
 struct ImpKind {
   int wp, we, wf;
@@ -223,11 +225,11 @@ KD_INL bool imp_conv_rel(const koral_params &P, int whicheq, double EPS, const d
 // the residual at the iterate (stage 0), the four Jacobian columns (1..4), a
 // damped trial (5) and the completion of a converged iterate (6).  The lanes
 // of a wave hold cells at different points of their iterations, so in
-// imp_newton_step's nested loops a wave waits for the lane with the most
-// damped trials (up to eleven) and repeated columns; here every lane advances
+// nested loops over iterations, columns and trials a wave waits for the lane
+// with the most damped trials (up to eleven) and repeated columns; here every lane advances
 // by one evaluation per trip whatever the others do, and the kernel holds one
 // inlined copy of the evaluation instead of four.  The operations on a cell
-// are those of imp_newton_step repeated, in the same order.
+// are those of the nested loops, in the same order.
 struct ImpLane {
   int stage, iter;
   double sign, xp, xj, xiapp, errbase;
@@ -291,7 +293,7 @@ KD_INL int imp_lane_trip(const koral_params &P, ImpLane &s, double *pp, const UT
         base = imp_trial_residual(WP, WE);
       }
     } else {
-      // a NaN factor ends the attempt too, as in imp_newton_step
+      // a NaN factor ends the attempt too
       if (!(s.xiapp >= P.maxradimpdamping)) return IMP_FAIL;
       update = true;
     }
@@ -343,7 +345,7 @@ KD_INL int imp_lane_trip(const koral_params &P, ImpLane &s, double *pp, const UT
 #if KD_WAVE_SOLVER
 // One attempt of a cell by a whole wave (solve_implicit_lab_4dprim from the
 // iterate pp, every argument the same in all lanes): the arithmetic and the
-// outcome of imp_newton_step repeated, bit for bit.  The wave is eight groups
+// outcome of the one-lane attempt, bit for bit.  The wave is eight groups
 // of eight lanes.  Group 0 evaluates the residual at the iterate while groups
 // 1..4 evaluate the four Jacobian columns (groups 5..7 repeat the iterate),
 // so an iteration costs one residual and one trial in sequence instead of
@@ -467,7 +469,7 @@ KD_INL int imp_wave_attempt(const koral_params &P, ImpKind k, WaveCell<MAG> &w, 
         wave_sync();
         continue;
       }
-      // a NaN factor ends the attempt too, as in imp_newton_step
+      // a NaN factor ends the attempt too
       if (!(xiapp >= P.maxradimpdamping)) return IMP_FAIL;
     }
     wave_sync();

@@ -1480,7 +1480,7 @@ struct GridTune {
                         // (OpSweep), 0 face states through HBM (OpRecon + OpFlux)
   int floor_wave;       // deferred passes: 1 a group of WAVE_GROUP lanes per face or cell, 0 one lane
   int update_pre;       // update: 1 the cell's u and p loaded with the fluxes
-  int comb_nv;          // 1: stage algebra with the variable count a template parameter
+  int comb_nv;          // 1: stage algebra in the launch of the u2p that follows, its variable count a template parameter
   int u2p_budget;       // OpU2P::budget
   int u2p_group;        // lanes per cell of the wave-mapped deferred u2p pass (64 or 32)
   long floor_nw;        // waves (or lanes) in flight in the deferred face passes
