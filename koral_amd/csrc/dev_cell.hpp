@@ -974,25 +974,90 @@ KD_FUN int floors_rad(const koral_params &P, double *pp, const Geom &g)
 // or CP_DEFERRED before writing uu (pp may be changed) and is redone by the
 // caller with DEFER false, with skip_hot for CP_DEFERRED_HOT.
 constexpr int CP_DEFERRED = 100, CP_DEFERRED_HOT = 101;
+struct CpFlags {
+  int entr, entr2, hd, rad;
+};
+// the flags of an inversion
+KD_INL CpFlags cp_flags(const int *corrected, const int *fixups)
+{
+  return CpFlags{corrected[0] == 1, corrected[2] == 1, fixups[0] > 0, fixups[1] > 0 ? -1 : 0};
+}
+// what follows the inversion: the floors, and uu from the floored
+// primitives.  DEFER: false, with uu untouched, where the b^2/rho floor is needed.
+template <int MAG, int RAD, bool DEFER, bool WAVE, int WG>
+KD_INL bool cp_floors(const koral_params &P, double *uu, double *pp, const Geom &g)
+{
+  MhdKin kin;
+  if (floors_mhd<MAG, RAD, DEFER, WAVE, WG>(P, pp, g, kin) == FLOORS_DEFERRED && DEFER) return false;
+  if (RAD) floors_rad<MAG, RAD>(P, pp, g);
+  p2u_mhd<MAG, RAD>(P, pp, uu, g, kin);
+  if (RAD) p2u_rad<MAG, RAD>(pp, uu, g);
+  return true;
+}
 template <int MAG, int RAD, bool DEFER = false, bool WAVE = false, int WG = WAVE_GROUP>
 KD_FUN int calc_primitives(const koral_params &P, double *uu, double *pp, const Geom &g, int &fl_entr,
                                int &fl_entr2, int &fl_hd, int &fl_rad, int budget = 0, bool skip_hot = false)
 {
   int corrected[3] = {0, 0, 0}, fixups[2] = {0, 0};
-  fl_entr = 0;
-  fl_entr2 = 0;
-  int r = u2p<MAG, RAD, DEFER, WAVE, WG>(P, uu, pp, g, corrected, fixups, budget, skip_hot);
+  const int r = u2p<MAG, RAD, DEFER, WAVE, WG>(P, uu, pp, g, corrected, fixups, budget, skip_hot);
   if (DEFER && r == U2P_DEFERRED) return CP_DEFERRED_HOT;
   if (DEFER && r == U2P_DEFERRED_105) return CP_DEFERRED;
-  if (corrected[0] == 1) fl_entr = 1;
-  if (corrected[2] == 1) fl_entr2 = 1;
-  MhdKin kin;
-  if (floors_mhd<MAG, RAD, DEFER, WAVE, WG>(P, pp, g, kin) == FLOORS_DEFERRED && DEFER) return CP_DEFERRED;
-  if (RAD) floors_rad<MAG, RAD>(P, pp, g);
-  p2u_mhd<MAG, RAD>(P, pp, uu, g, kin);
-  if (RAD) p2u_rad<MAG, RAD>(pp, uu, g);
-  fl_hd = (fixups[0] > 0) ? 1 : 0;
-  fl_rad = (fixups[1] > 0) ? -1 : 0;
+  if (!cp_floors<MAG, RAD, DEFER, WAVE, WG>(P, uu, pp, g)) return CP_DEFERRED;
+  const CpFlags f = cp_flags(corrected, fixups);
+  fl_entr = f.entr;
+  fl_entr2 = f.entr2;
+  fl_hd = f.hd;
+  fl_rad = f.rad;
+  return r;
+}
+
+// calc_primitives of a point by one lane, for a kernel that takes a whole
+// batch: the common path (hot inversion, floors without the b^2/rho one) and
+// the rare one after it, so that the rare path's inversions do not sit in the
+// common path's registers.  Each inversion runs once: a point at the b^2/rho
+// floor goes on from its inverted primitives, and a point whose hot inversion
+// failed with its guess left as it was starts at the entropy inversion.
+// load_g(g) reads the point's metric, load_s(uu, pp) its state; the rare path
+// reads them again rather than hold them over the common path, but for the
+// metric with field and radiation, whose kernel has one wave per SIMD and the
+// registers for it (a tenth of 2^20 points at the floor: 580 us, 584 reading it
+// again).  2^20 magnetised points, none and a tenth of them at the floor: 230
+// and 370 us; with both paths in one 335 and 510; with the rare path begun from
+// the inputs again 245 and 530.
+template <int MAG, int RAD, class LG, class LS>
+KD_INL int calc_primitives_point(const koral_params &P, LG &&load_g, LS &&load_s, double *uu, double *pp, CpFlags &fl)
+{
+  int corrected[3] = {0, 0, 0}, fixups[2] = {0, 0};
+  int r;
+  double rho = 0., u = 0.;  // inverted, before the floors
+  bool redo, done = false;
+  Geom g;
+  {
+    load_g(g);
+    load_s(uu, pp);
+    r = u2p<MAG, RAD, true>(P, uu, pp, g, corrected, fixups);
+    redo = r == U2P_DEFERRED || r == U2P_DEFERRED_105;
+    if (!redo) {
+      rho = pp[0];
+      u = pp[1];
+      done = cp_floors<MAG, RAD, true, false, WAVE_GROUP>(P, uu, pp, g);
+    }
+  }
+  if (!done) {
+    if (!(MAG && RAD)) {
+      compiler_fence();
+      load_g(g);
+    }
+    if (redo) {
+      load_s(uu, pp);
+      r = u2p<MAG, RAD>(P, uu, pp, g, corrected, fixups, 0, r == U2P_DEFERRED);
+    } else {
+      pp[0] = rho;
+      pp[1] = u;
+    }
+    cp_floors<MAG, RAD, false, false, WAVE_GROUP>(P, uu, pp, g);
+  }
+  fl = cp_flags(corrected, fixups);
   return r;
 }
 

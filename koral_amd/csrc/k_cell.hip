@@ -38,13 +38,8 @@ __global__ void __launch_bounds__(256) k_p2u(koral_params P, long n, const doubl
   for (int v = 0; v < NV; v++) uu[v * n + i] = u[v];
 }
 
-// calc_primitives per point.  The common path carries the hot inversion alone
-// and fits two waves per SIMD; a wave with points that need the entropy
-// inversion or the b^2/rho floor goes on with those lanes in the full path,
-// from their inputs again (entropy only where the hot inversion failed and
-// left the guess as it was): the path the point would have taken, so the same
-// result.  With both in one path the kernel took 364 registers, one wave per
-// SIMD.
+// calc_primitives per point, common and rare path in one launch
+// (calc_primitives_point).
 template <int MAG, int RAD>
 __global__ void __launch_bounds__(256, RAD && MAG ? 1 : 2) k_u2p(koral_params P, long n, double *__restrict__ uu,
                                                 double *__restrict__ pp, const double *__restrict__ g20,
@@ -55,36 +50,26 @@ __global__ void __launch_bounds__(256, RAD && MAG ? 1 : 2) k_u2p(koral_params P,
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   double p[NV], u[NV];
-  int fe, fe2, fh, fr, r;
-  auto load = [&](Geom &g) {
-    load_point<MAG, RAD>(g20, G20, n, i, g);
+  CpFlags fl;
+  ret[i] = calc_primitives_point<MAG, RAD>(
+      P, [&](Geom &g) { load_point<MAG, RAD>(g20, G20, n, i, g); },
+      [&](double *us, double *ps) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      p[v] = pp[v * n + i];
-      u[v] = uu[v * n + i];
-    }
-  };
-  {
-    Geom g;
-    load(g);
-    r = calc_primitives<MAG, RAD, true>(P, u, p, g, fe, fe2, fh, fr);
-  }
-  if (r == CP_DEFERRED || r == CP_DEFERRED_HOT) {
-    compiler_fence();
-    Geom g;
-    load(g);
-    r = calc_primitives<MAG, RAD>(P, u, p, g, fe, fe2, fh, fr, 0, r == CP_DEFERRED_HOT);
-  }
+        for (int v = 0; v < NV; v++) {
+          ps[v] = pp[v * n + i];
+          us[v] = uu[v * n + i];
+        }
+      },
+      u, p, fl);
 #pragma unroll
   for (int v = 0; v < NV; v++) {
     pp[v * n + i] = p[v];
     uu[v * n + i] = u[v];
   }
-  ret[i] = r;
-  flags[F_ENTROPY * n + i] = fe;
-  flags[F_ENTROPY2 * n + i] = fe2;
-  flags[F_HDFIXUP * n + i] = fh;
-  flags[F_RADFIXUP * n + i] = fr;
+  flags[F_ENTROPY * n + i] = fl.entr;
+  flags[F_ENTROPY2 * n + i] = fl.entr2;
+  flags[F_HDFIXUP * n + i] = fl.hd;
+  flags[F_RADFIXUP * n + i] = fl.rad;
 }
 
 // the W inversion from a learned W start (W0[i] > 0), retried from the
