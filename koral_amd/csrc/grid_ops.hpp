@@ -1501,14 +1501,20 @@ inline GridTune default_tune()
   return t;
 }
 
-// The choices a new grid starts with.  On a magnetised grid with MP5 the
-// fused sweep saves the face states' round trip through HBM where the box is
-// large enough to fill the chip with its 168-register waves: 128x128x64 zones
-// 3.08 ms per step split, 2.78 fused in all directions; 39 600 zones are
-// faster with only the x2 sweep fused, 2-D ones too.  The other
-// reconstructions spill in the fused kernel.  The update's early loads
-// (update_pre) are never slower, 128x128x64 2.78 -> 2.68 ms, and 64-thread
-// blocks suit the face kernels, 2.68 -> 2.60 ms.
+// The choices a new grid starts with (us per step, from the initial state /
+// from step 30).  On a magnetised grid with MP5 the fused sweep saves the face
+// states' round trip through HBM: split, x2 only and all directions fused take
+// 2883/3716, 2786/3644 and 2569/3592 on 128x128x64 zones, 963/1227, 896/1171
+// and 865/1165 on 96x64x24, and in 2-D 727/1338, 675/1294 and 669/1285 on
+// 400x256, 1948/2263, 1872/2183 and 1791/2105 on 1024x768.  Below the line the
+// two fused choices change places with the state: 80x64x19 866/1237, 807/1185
+// and 784/1212; 256x200 661/870, 609/827 and 606/817.  The other
+// reconstructions spill in the fused kernel.  Blocks of 64 threads against 256
+// for the face kernels: 7779/8657 and 7887/8736 on 192x192x96, 2569/3592 and
+// 2647/3579 on 128x128x64, 1038/1667 and 1010/1690 on 128x64x32, within 1 % in
+// 2-D.  The update's early loads (update_pre) were faster on every grid tried,
+// 1-D radiation tubes of 64 to 400 000 zones, 2-D and 3-D ones with each
+// reconstruction, by 2 to 6 %.
 inline GridTune grid_tune(const koral_params &P, const DGrid &G)
 {
   GridTune t = default_tune();
@@ -1535,7 +1541,8 @@ struct GridBufs {
   unsigned char *uwhy;  // per ulist entry: the redo may skip the failed hot inversion
   double *pn, *un;
   int *mark;
-  double *ut0, *ut1, *uforget, *dut1, *dut2, *drt1, *drt2;  // (dut2 is not stored: step_rk2imex)
+  // dut2 has no memory of its own (dut1's address): the launch that forms it is the only one to read it
+  double *ut0, *ut1, *uforget, *dut1, *dut2, *drt1, *drt2;
   double *tsd;    // time-step density max (one double)
   double *clock;  // {t, dt} of the operators (device scalars)
   int *counters;  // step counters [6]
@@ -1584,7 +1591,7 @@ void grid_buffers(GridBufs &s, F &&f)
   f(s.ut1, nv * nc, "ut1");
   f(s.uforget, nv * nc, "uforget");
   f(s.dut1, nv * nc, "dut1");
-  f(s.dut2, nv * nc, "dut2");
+  s.dut2 = s.dut1;
   f(s.drt1, nv * nc, "drt1");
   f(s.drt2, nv * nc, "drt2");
   f(s.tsd, 1L, "tstepden");
