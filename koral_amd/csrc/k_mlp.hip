@@ -630,7 +630,7 @@ __global__ void __launch_bounds__(64 * INFER_WAVES, 4) k_mlp_infer(const unsigne
         h[t][ot] = activate(acc, sb, ot);
       }
     }
-    // layers 2 and 3: one copy of the code (it holds 64 inlined tanh)
+    // layers 2 and 3: one copy of the code (it holds 32 inlined tanh)
 #pragma unroll 1
     for (int layer = 0; layer < 2; layer++) {
       bf16x4 hn[CT][NH / 16];
