@@ -187,8 +187,11 @@ KD_INL double Sfromu(const koral_params &P, double rho, double u)
 }
 
 // Four-velocity and magnetic four-vector of a primitive state: functions of
-// its velocities and field alone, which the floors, the conserved state and
-// the fluxes of one state share
+// its velocities and field alone, which the floors and the conserved state
+// that follows them share in calc_primitives.  The faces do not: holding them
+// over a side's floors, flux and conserved state cost the sweeps 8 to 14 more
+// spilled registers (six fused sweeps of 128x128x64 zones 0.86 -> 0.91 ms, six
+// flux kernels of split ones 0.67 -> 0.76 ms).
 struct MhdKin {
   double ucon[4], ucov[4], bcon[4], bcov[4], bsq;
 };

@@ -221,12 +221,17 @@ KD_INL void ppm(const double *v, const double *dx, double &ul, double &ur)
 
 // ---- physical fluxes ----
 template <int MAG, int RAD>
-KD_INL void flux_prime(const koral_params &P, const double *pp, int d, const Geom &g, const MhdKin &k, double *ff)
+KD_INL void flux_prime(const koral_params &P, const double *pp, int d, const Geom &g, double *ff)
 {
   constexpr int EE = Lay<MAG, RAD>::EE;
-  const double *ucon = k.ucon, *ucov = k.ucov, *bcon = k.bcon, *bcov = k.bcov;
-  const double bsq = k.bsq;
   double gdetu = g.gdet;
+  double ucon[4], ucov[4], bcon[4] = {0., 0., 0., 0.}, bcov[4] = {0., 0., 0., 0.}, bsq = 0.;
+  relr_to_4vel(pp[2], pp[3], pp[4], ucon, ucov, g);
+  if (MAG) {
+    bcon4(pp[6], pp[7], pp[8], ucon, ucov, bcon);
+    lower(bcon, bcov, g);
+    bsq = dot4(bcon, bcov);
+  }
   double rho = pp[0], u = pp[1], S = pp[5];
   double pre = (P.gamma - 1.) * u;
   double w = rho + u + pre;

@@ -541,26 +541,20 @@ struct OpReconRun {
   }
 };
 
-// Physical flux and conserved state of one side of a face, from its floored
-// state p and k = mhd_kin of it
-template <int MAG, int RAD, int D>
-KD_INL void face_side(const koral_params &P, const double *p, const Geom &g, const MhdKin &k, double *f, double *u)
-{
-  flux_prime<MAG, RAD>(P, p, D + 1, g, k, f);
-  p2u_mhd<MAG, RAD>(P, p, u, g, k);
-  if (RAD) p2u_rad<MAG, RAD>(p, u, g);
-}
-
-// HLL or LF at the face (ix, iy, iz) of direction D from the fluxes and
-// conserved states of its sides, with the wave speeds of the two cells
-// (f_calc_fluxes_at_faces finite.c:1297-1415)
+// Fluxes at the face (ix, iy, iz) of direction D from its floored face
+// states: physical fluxes, conserved states, HLL or LF with the wave speeds
+// of the two cells (f_calc_fluxes_at_faces finite.c:1297-1415)
 template <int MAG, int RAD, int D>
 KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
-                      int iy, int iz, const double *fL, const double *uL, const double *fR, const double *uR,
-                      bool store = true)
+                      int iy, int iz, const double *pL, const double *pR, const Geom &g, bool store = true)
 {
   constexpr int NV = Lay<MAG, RAD>::NV;
   constexpr int NVMHD = 6 + 3 * MAG;
+  double fL[NV], fR[NV], uL[NV], uR[NV];
+  flux_prime<MAG, RAD>(P, pL, D + 1, g, fL);
+  flux_prime<MAG, RAD>(P, pR, D + 1, g, fR);
+  kd::p2u<MAG, RAD>(P, pL, uL, g);
+  kd::p2u<MAG, RAD>(P, pR, uR, g);
   const long n = G.ncell;
   const long cR = cidx(G, ix, iy, iz), cL = cR - dir_stride<D>(G);
   const long f = fidx(G, D, ix, iy, iz);
@@ -584,49 +578,6 @@ KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__res
     }
     if (store) flb[iv * nf + f] = F;
   }
-}
-
-// the same from the floored states
-template <int MAG, int RAD, int D>
-KD_INL void face_flux(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
-                      int iy, int iz, const double *pL, const double *pR, const Geom &g, bool store = true)
-{
-  constexpr int NV = Lay<MAG, RAD>::NV;
-  double fL[NV], uL[NV], fR[NV], uR[NV];
-  MhdKin k;
-  mhd_kin<MAG>(pL, g, k);
-  face_side<MAG, RAD, D>(P, pL, g, k, fL, uL);
-  mhd_kin<MAG>(pR, g, k);
-  face_side<MAG, RAD, D>(P, pR, g, k, fR, uR);
-  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, fL, uL, fR, uR, store);
-}
-
-// The common path of a face from its two states: floors, fluxes, Riemann
-// solver, one side after the other (the four-vectors of a side serve its
-// floors, flux and conserved state and are gone before the other's).  Returns
-// true, with nothing stored, when a state needs the b^2/rho floor.
-template <int MAG, int RAD, int D>
-KD_INL bool face_common(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
-                        int iy, int iz, double *pL, double *pR, const Geom &g, unsigned i, unsigned *list,
-                        unsigned *cnt)
-{
-  constexpr int NV = Lay<MAG, RAD>::NV;
-  double fL[NV], uL[NV], fR[NV], uR[NV];
-  bool defer;
-  {
-    MhdKin k;
-    defer = floors_mhd<MAG, RAD, true>(P, pL, g, k) == FLOORS_DEFERRED;
-    face_side<MAG, RAD, D>(P, pL, g, k, fL, uL);
-  }
-  {
-    MhdKin k;
-    if (floors_mhd<MAG, RAD, true>(P, pR, g, k) == FLOORS_DEFERRED) defer = true;
-    face_side<MAG, RAD, D>(P, pR, g, k, fR, uR);
-  }
-  append_index(defer, i, list, cnt);
-  if (defer) return true;
-  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, fL, uL, fR, uR);
-  return false;
 }
 
 // face states of face i of a sweep box, stored by OpRecon
@@ -668,7 +619,12 @@ struct OpFlux {
     load_face_states<NV>(fs, b.size(), i, pL, pR);
     Geom g;
     geom_face(G, D, ix, iy, g);
-    face_common<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, (unsigned)i, list, cnt);
+    const int dl = floors_mhd<MAG, RAD, true>(P, pL, g);
+    const int dr = floors_mhd<MAG, RAD, true>(P, pR, g);
+    const bool defer = dl == FLOORS_DEFERRED || dr == FLOORS_DEFERRED;
+    append_index(defer, (unsigned)i, list, cnt);
+    if (defer) return;
+    face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g);
   }
 };
 
@@ -711,15 +667,6 @@ KD_INL void floors_pair(const koral_params &P, double *pL, double *pR, const Geo
   }
 }
 
-// The rare path: the full floors on both states, then the same fluxes
-template <int MAG, int RAD, int D, bool WAVE>
-KD_INL void face_floored(const koral_params &P, const DGrid &G, const double *__restrict__ ws, double *flb, int ix,
-                         int iy, int iz, double *pL, double *pR, const Geom &g, bool store)
-{
-  floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
-  face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, store);
-}
-
 // The faces OpFlux left: the same face states, the full face floors, the
 // same fluxes.  WAVE: a group of WAVE_GROUP lanes per face (the floors' W
 // inversions evaluate their trials one per lane; the group's first lane
@@ -750,7 +697,8 @@ struct OpFluxFloor {
       load_face_states<NV>(fs, b.size(), i, pL, pR);
       Geom g;
       geom_face(G, D, ix, iy, g);
-      face_floored<MAG, RAD, D, WAVE>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
+      floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
+      face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
     }
   }
 };
@@ -803,7 +751,12 @@ struct OpSweep {
     face_states<MAG, RAD, ORDER, D>(P, G, p, ix, iy, iz, pL, pR);
     Geom g;
     geom_face(G, D, ix, iy, g);
-    face_common<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, (unsigned)i, list, cnt);
+    const int dl = floors_mhd<MAG, RAD, true>(P, pL, g);
+    const int dr = floors_mhd<MAG, RAD, true>(P, pR, g);
+    const bool defer = dl == FLOORS_DEFERRED || dr == FLOORS_DEFERRED;
+    append_index(defer, (unsigned)i, list, cnt);
+    if (defer) return;
+    face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g);
   }
 };
 
@@ -834,7 +787,8 @@ struct OpSweepFloor {
       face_states<MAG, RAD, ORDER, D>(P, G, p, ix, iy, iz, pL, pR);
       Geom g;
       geom_face(G, D, ix, iy, g);
-      face_floored<MAG, RAD, D, WAVE>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
+      floors_pair<MAG, RAD, WAVE>(P, pL, pR, g);
+      face_flux<MAG, RAD, D>(P, G, ws, flb, ix, iy, iz, pL, pR, g, lead);
     }
   }
 };
@@ -1504,14 +1458,14 @@ inline GridTune default_tune()
 // The choices a new grid starts with (us per step, from the initial state /
 // from step 30).  On a magnetised grid with MP5 the fused sweep saves the face
 // states' round trip through HBM: split, x2 only and all directions fused take
-// 2883/3716, 2786/3644 and 2569/3592 on 128x128x64 zones, 963/1227, 896/1171
-// and 865/1165 on 96x64x24, and in 2-D 727/1338, 675/1294 and 669/1285 on
-// 400x256, 1948/2263, 1872/2183 and 1791/2105 on 1024x768.  Below the line the
-// two fused choices change places with the state: 80x64x19 866/1237, 807/1185
-// and 784/1212; 256x200 661/870, 609/827 and 606/817.  The other
+// 2796/3647, 2685/3528 and 2512/3529 on 128x128x64 zones, 954/1212, 895/1155
+// and 863/1149 on 96x64x24, and in 2-D 654/1062, 587/1000 and 578/989 on
+// 400x256, 1905/2222, 1816/2123 and 1739/2060 on 1024x768.  Below the line the
+// two fused choices change places with the state: 80x64x19 859/1232, 794/1178
+// and 772/1195; 256x200 655/868, 604/812 and 600/813.  The other
 // reconstructions spill in the fused kernel.  Blocks of 64 threads against 256
-// for the face kernels: 7779/8657 and 7887/8736 on 192x192x96, 2569/3592 and
-// 2647/3579 on 128x128x64, 1038/1667 and 1010/1690 on 128x64x32, within 1 % in
+// for the face kernels: 7592/8437 and 7641/8500 on 192x192x96, 2512/3529 and
+// 2585/3503 on 128x128x64, 1017/1643 and 995/1656 on 128x64x32, within 1 % in
 // 2-D.  The update's early loads (update_pre) were faster on every grid tried,
 // 1-D radiation tubes of 64 to 400 000 zones, 2-D and 3-D ones with each
 // reconstruction, by 2 to 6 %.
