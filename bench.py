@@ -34,11 +34,12 @@ FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 (vector and matrix)
 # FETCH_SIZE and WRITE_SIZE per dispatch scaled by the same counters on a
 # streaming kernel of known size (profiles/hbm_traffic_grmhd_torus_128x128x64.md).
 # The face kernels per sweep direction (x1, x2, x3) and schedule (None: not
-# measured); the update per variant (tune.update_pre).
+# measured); the update per variant (tune.update_pre); u2p with the stage
+# algebra in its launch (tune.comb_nv), the mean of a step's four launches.
 GRID_TRAFFIC_128x128x64 = {
-    "u2p": 315e6,
-    "update": {1: 581e6},
-    "flux": {"split": (None, None, None), "fused": (448e6, 880e6, 398e6)},
+    "u2p": {1: 550e6},
+    "update": {1: 524e6},
+    "flux": {"split": (None, None, None), "fused": (431e6, 864e6, 398e6)},
     "recon": {"split": (None, None, None)},
 }
 
@@ -386,14 +387,18 @@ def cpu_baseline_implicit(P, pp, g20, G20, dt, args):
 # primitive/conserved vector is one NV-vector of FP64; stencil neighbours are
 # shared through the caches; the metric lives in per-(x1, x2) tables read
 # through the caches by every x3 column (no per-unit HBM bytes).
-def grid_alg_bytes(kind, nv, fused=False):
+def grid_alg_bytes(kind, nv, fused=False, algebra=False, mag=False):
+    nb = 3 if mag else 0                           # field fluxes: three EMFs stand for them in the update
     return {
         "recon": (nv + 2 * nv) * 8,                # per face: prims of its cell, both face states
         # per face: face states (split) or cell prims (fused), 3 wave-speed
         # values (each cell's shared by its two faces), the flux
         "flux": ((nv if fused else 2 * nv) + 3 + nv) * 8,
-        "u2p": (4 * nv) * 8 + 4,                   # per cell: u, p in and out, 4 flag bytes
-        "update": (nv + nv + 3 * nv + nv) * 8,     # per cell: p, u, 3 face fluxes, u
+        # per cell: u, p in and out, 4 flag bytes; with the stage algebra in
+        # the launch the mean of a step's four (without radiation): p in and
+        # out, u out, and 2, 4, 4 and 5 arrays read or written by the algebra
+        "u2p": ((3 + 15 / 4) * nv if algebra else 4 * nv) * 8 + 4,
+        "update": (nv + nv + 3 * (nv - nb) + nb + nv) * 8,  # per cell: p, u, 3 face fluxes, u
         "wavespeeds": (nv + 18) * 8,               # per cell: prims, 18 speeds
         "emf": 9 * 8, "ct_faces": 9 * 8,           # per edge
         "comb": 3 * 8,                             # per (cell, variable)
@@ -510,7 +515,7 @@ def bench_grid(args, kind):
     if dom == "flux":
         bpu = sum(grid_alg_bytes("flux", P.nv, bool(tn.fused[d])) for d in dims) / len(dims)
     else:
-        bpu = grid_alg_bytes(dom, P.nv)
+        bpu = grid_alg_bytes(dom, P.nv, algebra=bool(tn.comb_nv), mag=bool(P.mag))
     bytes_launch = bpu * units / nl
     achieved = bytes_launch / per_launch / 1e9
     traffic = None
@@ -521,11 +526,11 @@ def bench_grid(args, kind):
             traffic = sum(v) / len(v) if None not in v else None
         elif dom == "update":
             traffic = tr.get(tn.update_pre)
+        elif dom == "u2p":
+            traffic = tr.get(tn.comb_nv)
         elif dom == "recon":
             v = [tr["split"][d] for d in dims if not tn.fused[d]]
             traffic = sum(v) / len(v) if v and None not in v else None
-        elif isinstance(tr, float):
-            traffic = tr
     # FP64 rate of the dominant kernel from the operation count (the face
     # kernels only when every sweep is fused: a split sweep's flux kernel
     # does not do the reconstruction the count includes)
