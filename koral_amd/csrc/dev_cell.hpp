@@ -339,7 +339,8 @@ KD_INL bool w_bad(double W, double Bsq, double QdotBsq, double Qtsq)
 // Wstart > 0 replaces the W start computed from pp (the learned W guess,
 // which has no reference counterpart); iters, when given, receives the
 // Newton iterations made.  budget > 0 (sequential path only) bounds the
-// residual evaluations: the solver gives up with U2P_OVER_BUDGET, pp
+// residual evaluations, a trial or four halvings rejected without one
+// counting an eighth: the solver gives up with U2P_OVER_BUDGET, pp
 // untouched, when a point needs more (a caller that can hand the point to
 // the wave-parallel solver redoes it there from the start, same result).
 // entropy false: pp[5] is left as it was (a caller that does not read it
@@ -492,7 +493,7 @@ KD_FUN int u2p_solver_W(const koral_params &P, const double *uu, double *pp, con
         Wt = m == 0 ? t[0] : m == 1 ? t[1] : m == 2 ? t[2] : t[3];
       }
       nev += 8;
-      if (budget > 0 && nev > 8 * budget) return U2P_OVER_BUDGET;
+      if (budget > 0 && (nev - 1) / 8 >= budget) return U2P_OVER_BUDGET;
       f_u2p(P, etype, Wt - D, c, f, df, e);
       ok = phase == MOVED || (isfinite(f) && isfinite(df));
     }
