@@ -153,9 +153,10 @@ class Net:
         X [11][N], T [4][N] (device).  Returns the mean loss of each epoch
         (from every 64th batch)."""
         N = X.shape[1]
-        if X.shape[0] < NIN or T.shape[0] < NOUT or T.shape[1] < N:
-            raise ValueError("expected X [%d][N] and T [%d][N]" % (NIN, NOUT))
-        X, T = _chk(X.contiguous(), torch.float32), _chk(T[:, :N].contiguous(), torch.float32)
+        if N >= batch:
+            if X.shape[0] < NIN or T.shape[0] < NOUT or T.shape[1] < N:
+                raise ValueError("expected X [%d][N] and T [%d][N]" % (NIN, NOUT))
+            X, T = _chk(X.contiguous(), torch.float32), _chk(T[:, :N].contiguous(), torch.float32)
         gen = torch.Generator(device=X.device)
         gen.manual_seed(seed)
         hist = []
