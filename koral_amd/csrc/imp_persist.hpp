@@ -83,6 +83,10 @@ struct ImpBufs {
 // against 24.5 ms by the passes, 10 000 cells 18.4 against 25.3 ms, 20 000
 // cells 28.6 against 26.1 ms).
 constexpr long IMP_WAVE_CELLS = 1L << 14;
+// the line of the kernels without scratch (implicit_passes), which hold half
+// the waves at a time: 12 288 cells 22.5 ms by waves, 12 289 cells 25.0 by the
+// passes, 16 384 cells 28 by the passes
+constexpr long IMP_WAVE_CELLS_NOSCRATCH = 3L << 12;
 
 // pass modes of k_imp_pass
 enum { IMP_CHAIN = 0, IMP_LEARN1 = 1, IMP_LEARN2 = 2 };
@@ -384,9 +388,10 @@ __global__ void __launch_bounds__(256) k_imp_finish(koral_params P, Src src, lon
 
 // The whole chain of n cells, a wave per cell: a cell's attempts follow one
 // another in its wave, so the time of a launch with few cells is one cell's
-// chain.
-template <int MAG, class Src>
-__global__ void __launch_bounds__(256, 2) k_imp_wave(koral_params P, Src src, int *counts, const double *gxg,
+// chain.  Two waves per SIMD (WPS) spill 430 bytes a lane and are still faster
+// than one without spills (7.4 against 9.7 ms for 3001 cells).
+template <int MAG, int WPS, class Src>
+__global__ void __launch_bounds__(256, WPS) k_imp_wave(koral_params P, Src src, int *counts, const double *gxg,
                                                      const double *gxr, long n, int learned_maxiter)
 {
   constexpr int NV = Lay<MAG, 1>::NV;
@@ -479,10 +484,10 @@ __global__ void __launch_bounds__(256, 2) k_imp_wave(koral_params P, Src src, in
 }
 
 // clears n (<= 64) counters on the launching stream (a kernel, so the clear
-// can sit inside a captured graph)
-static __global__ void k_zero_u32(unsigned *q, int n)
+// can sit inside a captured graph), and sets counter one (>= 0) to 1
+static __global__ void k_zero_u32(unsigned *q, int n, int one)
 {
-  if ((int)threadIdx.x < n) q[threadIdx.x] = 0u;
+  if ((int)threadIdx.x < n) q[threadIdx.x] = (int)threadIdx.x == one ? 1u : 0u;
 }
 
 // Blocks of bs threads that fill every CU at the kernel's occupancy (never
@@ -507,16 +512,18 @@ int resident_blocks(K kernel, int bs, long n, unsigned *blocks)
 // sooner with the SIMDs to themselves (measured: 262 144 cells 37.1 against
 // 38.9 ms, 2^20 cells 75.2 against 65.0 ms with one and two blocks a CU).
 constexpr long IMP_TWO_BLOCKS = 1L << 19;
-template <int MAG, int WE, int WF, int MODE = IMP_CHAIN, class Src>
+template <int MAG, bool SCRATCH, int WE, int WF, int MODE = IMP_CHAIN, class Src>
 int imp_launch_pass(const koral_params &P, const Src &src, long n, int a, const ImpBufs &b, int *counts,
                     hipStream_t s, const double *gxg = nullptr, const double *gxr = nullptr)
 {
   unsigned two = 0, one = 0;
-  int rc = resident_blocks(k_imp_pass<MAG, true, WE, WF, MODE, Src>, 256, n, &two);
-  if (!rc) rc = resident_blocks(k_imp_pass<MAG, false, WE, WF, MODE, Src>, 256, n, &one);
+  int rc = resident_blocks(k_imp_pass<MAG, false, WE, WF, MODE, Src>, 256, n, &one);
+  if constexpr (SCRATCH) {
+    if (!rc) rc = resident_blocks(k_imp_pass<MAG, true, WE, WF, MODE, Src>, 256, n, &two);
+    if (n < IMP_TWO_BLOCKS && two > one) two = one;
+    if (!rc) k_imp_pass<MAG, true, WE, WF, MODE, Src><<<two, 256, 0, s>>>(P, src, a, b, counts, gxg, gxr, n);
+  }
   if (rc) return rc;
-  if (n < IMP_TWO_BLOCKS && two > one) two = one;
-  k_imp_pass<MAG, true, WE, WF, MODE, Src><<<two, 256, 0, s>>>(P, src, a, b, counts, gxg, gxr, n);
   k_imp_pass<MAG, false, WE, WF, MODE, Src><<<one, 256, 0, s>>>(P, src, a, b, counts, gxg, gxr, n);
   return 0;
 }
@@ -526,37 +533,44 @@ int imp_launch_pass(const koral_params &P, const Src &src, long n, int a, const 
 // be null) the radiation start (E, F~^1..3); the learned pass stops a cell
 // after learned_maxiter iterations when that is positive and below
 // RADIMPMAXITER.
-template <int MAG, class Src>
+//
+// SCRATCH false: kernels that need no scratch memory alone, for a caller that
+// cannot have device memory taken (the runtime sets scratch aside when a queue
+// first runs a kernel that spills: 216 MiB for the wave kernel, 26 for the
+// passes).  These are the wave kernel at one wave per SIMD and the passes'
+// general variant, at one block a CU.
+template <int MAG, bool SCRATCH = true, class Src>
 int implicit_passes(const koral_params &P, const Src &src, long n, const ImpBufs &b, int *counts, hipStream_t s, const double *gxg = nullptr, const double *gxr = nullptr, int learned_maxiter = 0)
 {
   const unsigned nb = (unsigned)((n + 255) / 256);
   koral_params Pl = P;
   if (learned_maxiter > 0 && learned_maxiter < Pl.radimpmaxiter) Pl.radimpmaxiter = learned_maxiter;
   int rc = 0;
-  if (n <= IMP_WAVE_CELLS) {
+  if (n <= (SCRATCH ? IMP_WAVE_CELLS : IMP_WAVE_CELLS_NOSCRATCH)) {
+    constexpr int WPS = SCRATCH ? 2 : 1;
     unsigned blocks = 0;
-    rc = resident_blocks(k_imp_wave<MAG, Src>, 256, 64 * n, &blocks);
-    if (!rc) k_imp_wave<MAG, Src><<<blocks, 256, 0, s>>>(P, src, counts, gxg, gxr, n, Pl.radimpmaxiter);
+    rc = resident_blocks(k_imp_wave<MAG, WPS, Src>, 256, 64 * n, &blocks);
+    if (!rc) k_imp_wave<MAG, WPS, Src><<<blocks, 256, 0, s>>>(P, src, counts, gxg, gxr, n, Pl.radimpmaxiter);
     return rc;
   }
-  k_zero_u32<<<1, 64, 0, s>>>(b.ctr, IMP_NCTR);
+  k_zero_u32<<<1, 64, 0, s>>>(b.ctr, IMP_NCTR, SCRATCH ? -1 : IMP_ASYM);
   if (gxg) {
     k_imp_learned_classify<MAG, Src><<<nb, 256, 0, s>>>(P, src, n, b, gxg, gxr);
     // without a radiation guess there is no second try: b.second must then be null
     ImpBufs bl = b;
     if (!gxr) bl.second[0] = bl.second[1] = nullptr;
-    rc = imp_launch_pass<MAG, ENERGYEQ, LAB, IMP_LEARN1>(Pl, src, n, 0, bl, counts, s, gxg, gxr);
-    if (!rc && bl.second[0]) rc = imp_launch_pass<MAG, ENERGYEQ, LAB, IMP_LEARN2>(Pl, src, n, 0, bl, counts, s, gxg, gxr);
+    rc = imp_launch_pass<MAG, SCRATCH, ENERGYEQ, LAB, IMP_LEARN1>(Pl, src, n, 0, bl, counts, s, gxg, gxr);
+    if (!rc && bl.second[0]) rc = imp_launch_pass<MAG, SCRATCH, ENERGYEQ, LAB, IMP_LEARN2>(Pl, src, n, 0, bl, counts, s, gxg, gxr);
   } else {
     k_imp_classify<MAG, 1, Src><<<nb, 256, 0, s>>>(P, src, n, b);
   }
   for (int a = 0; a < 6 && !rc; a++) {
     if (a >= 4)
-      rc = imp_launch_pass<MAG, ENTROPYEQ, LAB>(P, src, n, a, b, counts, s);
+      rc = imp_launch_pass<MAG, SCRATCH, ENTROPYEQ, LAB>(P, src, n, a, b, counts, s);
     else if (a == 1 || a == 3)
-      rc = imp_launch_pass<MAG, ENERGYEQ, FF>(P, src, n, a, b, counts, s);
+      rc = imp_launch_pass<MAG, SCRATCH, ENERGYEQ, FF>(P, src, n, a, b, counts, s);
     else
-      rc = imp_launch_pass<MAG, ENERGYEQ, LAB>(P, src, n, a, b, counts, s);
+      rc = imp_launch_pass<MAG, SCRATCH, ENERGYEQ, LAB>(P, src, n, a, b, counts, s);
   }
   if (!rc) k_imp_finish<MAG, Src><<<nb, 256, 0, s>>>(P, src, n);
   return rc;

@@ -516,10 +516,10 @@ int koral_hip_implicit_batch_noalloc(const koral_params *P, long n, double *uu, 
   b.ctr = ptr + NOALLOC_LISTS;
   if (P->mag) {
     BatchCells<1, 1> src{n, uu, pp, g20, G20, dt, flags, info, global_time};
-    rc = implicit_passes<1>(*P, src, n, b, nullptr, s);
+    rc = implicit_passes<1, false>(*P, src, n, b, nullptr, s);
   } else {
     BatchCells<0, 1> src{n, uu, pp, g20, G20, dt, flags, info, global_time};
-    rc = implicit_passes<0>(*P, src, n, b, nullptr, s);
+    rc = implicit_passes<0, false>(*P, src, n, b, nullptr, s);
   }
   if (rc) return rc;
   return check_launch("koral_hip_implicit_batch_noalloc");
