@@ -1022,42 +1022,40 @@ KD_FUN int calc_primitives(const koral_params &P, double *uu, double *pp, const 
 // floor goes on from its inverted primitives, and a point whose hot inversion
 // failed with its guess left as it was starts at the entropy inversion.
 // load_g(g) reads the point's metric, load_s(uu, pp) its state; the rare path
-// reads them again rather than hold them over the common path, but for the
-// metric with field and radiation, whose kernel has one wave per SIMD and the
-// registers for it (a tenth of 2^20 points at the floor: 580 us, 584 reading it
-// again).  2^20 magnetised points, none and a tenth of them at the floor: 230
-// and 370 us; with both paths in one 335 and 510; with the rare path begun from
-// the inputs again 245 and 530.
+// reads them again rather than hold them over the common path.  2^20
+// magnetised points, none and a tenth of them at the floor: 199 and 345 us;
+// with both paths in one 310 and 494; with the rare path begun from the inputs
+// again 227 and 506.  With radiation as well 345 and 561; 367 and 552; 333 and
+// 756 (200 003 points: 86 and 138; 98 and 137; 86 and 183).  One Geom serves
+// both paths: with one each the magnetised points without floors took 310 us.
 template <int MAG, int RAD, class LG, class LS>
 KD_INL int calc_primitives_point(const koral_params &P, LG &&load_g, LS &&load_s, double *uu, double *pp, CpFlags &fl)
 {
   int corrected[3] = {0, 0, 0}, fixups[2] = {0, 0};
   int r;
-  double rho = 0., u = 0.;  // inverted, before the floors
   bool redo, done = false;
   Geom g;
-  {
-    load_g(g);
-    load_s(uu, pp);
-    r = u2p<MAG, RAD, true>(P, uu, pp, g, corrected, fixups);
-    redo = r == U2P_DEFERRED || r == U2P_DEFERRED_105;
-    if (!redo) {
-      rho = pp[0];
-      u = pp[1];
-      done = cp_floors<MAG, RAD, true, false, WAVE_GROUP>(P, uu, pp, g);
+  load_g(g);
+  load_s(uu, pp);
+  r = u2p<MAG, RAD, true>(P, uu, pp, g, corrected, fixups);
+  redo = r == U2P_DEFERRED || r == U2P_DEFERRED_105;
+  if (!redo) {
+    // the floors' test, before they change the primitives
+    if (MAG) {
+      MhdKin k;
+      mhd_kin<MAG>(pp, g, k);
+      done = !(k.bsq / 2. > P.b2rhoratiomax * (pp[0] < P.rhofloor ? P.rhofloor : pp[0]));
+    } else {
+      done = true;
     }
+    if (done) (void)cp_floors<MAG, RAD, true, false, WAVE_GROUP>(P, uu, pp, g);
   }
   if (!done) {
-    if (!(MAG && RAD)) {
-      compiler_fence();
-      load_g(g);
-    }
+    compiler_fence();
+    load_g(g);
     if (redo) {
       load_s(uu, pp);
       r = u2p<MAG, RAD>(P, uu, pp, g, corrected, fixups, 0, r == U2P_DEFERRED);
-    } else {
-      pp[0] = rho;
-      pp[1] = u;
     }
     cp_floors<MAG, RAD, false, false, WAVE_GROUP>(P, uu, pp, g);
   }

@@ -78,8 +78,8 @@ def test_host_points(oracle, exe, tmp_path, mag, rad):
     once = (hot >= 0) & (uu[:, 0] >= 0.)
     floored = once & floor
     assert np.all(oh[once, 5] == 1) and np.any(oh[:, 5] == 2)
-    # the rare path: with field and radiation it keeps the metric
-    assert np.all(oh[floored, 6] == (1 if rad else 2)) and (not mag or floored.sum() > n // 16)
+    # the rare path reads the metric again
+    assert np.all(oh[floored, 6] == 2) and (not mag or floored.sum() > n // 16)
 
 
 @pytest.mark.gpu
